@@ -324,8 +324,8 @@ int afmm_create(const afmm_params* prm, afmm_ctx** out) {
         AFMM_CHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         for (auto& e : c->ev) AFMM_CHECK(hipEventCreate(&e));
         const Tables& T = tables_for_order(prm->p);
-        const std::vector<double> m2m = mfma_a_layout(T.m2m, T.S, 8);
-        const std::vector<double> l2l = mfma_a_layout(T.l2l, T.S, 8);
+        const std::vector<double> m2m = level_a_layout(T.m2m, prm->p);
+        const std::vector<double> l2l = level_a_layout(T.l2l, prm->p);
         // M2L operators in slot order (the order the M2L kernels step through them)
         std::vector<double> m2l_slots(T.m2l.size());
         const size_t SS = (size_t)T.S * T.S;

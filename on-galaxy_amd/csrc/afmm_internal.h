@@ -229,8 +229,8 @@ struct FmmTimes {
     float upward = 0, m2l = 0, downward = 0, leaf = 0;
 };
 struct FmmTables {
-    const double *m2m_sw, *l2l_sw;  // device, 8 octant operators in the MFMA A-fragment layout
-    const double* m2l_sw;           // device, 343 offset operators in the same layout
+    const double *m2m_sw, *l2l_sw;  // device, octant-0 operators in class-major MFMA A fragments (level_a_layout)
+    const double* m2l_sw;           // device, 343 offset operators in MFMA A fragments (m2l_a_layout)
     const float2* m2l_hl;           // device, the same as FP32 (hi, lo) pairs, or null
     const uint4* m2l_bf;            // device, three-piece bf16 layout (mfma_bf16_layout), or null
 };

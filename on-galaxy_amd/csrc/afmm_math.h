@@ -304,16 +304,53 @@ constexpr M2LSlots make_m2l_slots() {
 }
 constexpr M2LSlots kM2LSlotsHost = make_m2l_slots();
 
-// M2L operator tiling for v_mfma_f64_16x16x4_f64: RB row blocks of 16 and the
-// k steps of 4 split into NKC chunks of KC steps, one chunk of all row blocks
-// (RB*KC*64 doubles, RB*KC <= 60) small enough to double-buffer in under
-// 64 KB of LDS.
+// ---- reflection classes ---------------------------------------------------------
+// Reflecting an axis maps every real coefficient to itself times +-1: x to -x
+// multiplies Re a_n^a by (-1)^a and Im a_n^a by -(-1)^a, y to -y flips Im, z to
+// -z multiplies both by (-1)^(n+a). The class of a coefficient holds its three
+// signs as bits (1, 2, 4 for x, y, z; set where the sign is -1), the octant bits
+// of the tree. With D_s the diagonal of the signs of a set s of axes, the
+// translation by a reflected offset is D_s T D_s, so the sum over the eight
+// octants (children of a parent) needs one operator T and not eight:
+//   sum_s D_s T D_s x_s has row r = sum_k T[r][k] W_{class(r) ^ class(k)}[k],
+//   W_q[k] = sum_s (-1)^|s & q| x_s[k],
+// a Walsh-Hadamard transform of the eight inputs and one S x S product.
+constexpr int kMaxTerms = nterms(kMaxOrder);
+AFMM_HD constexpr int sym_class(int n, int a, int im) { return ((a & 1) ^ im) | (im << 1) | (((n + a) & 1) << 2); }
+// Class-major order of the coefficients for 16x16x4 matrix steps, each class
+// padded to whole k steps of 4: krow[4 q + e] is the storage index of row e of
+// step q (-1: padding), kcls[q] the class of step q, cnt[c] the coefficients of
+// class c, kfirst[c] its first step. Degrees ascend inside a class.
+struct SymTab {
+    int nq = 0;           // k steps
+    int rb = 0;           // 16-row blocks of the largest class
+    int cnt[8] = {}, kfirst[9] = {};
+    short krow[4 * (kMaxTerms / 4 + 8)] = {};
+    signed char kcls[kMaxTerms / 4 + 8] = {};
+};
+constexpr SymTab make_sym_tab(int p) {
+    SymTab t{};
+    for (int c = 0; c < 8; ++c) {
+        t.kfirst[c] = t.nq;
+        int m = 0;
+        for (int n = 0; n <= p; ++n)
+            for (int a = 0; a <= n; ++a)
+                for (int im = 0; im < (a ? 2 : 1); ++im)
+                    if (sym_class(n, a, im) == c) t.krow[4 * t.nq + m++] = (short)(rid(n, a) + im);
+        t.cnt[c] = m;
+        if ((m + 15) / 16 > t.rb) t.rb = (m + 15) / 16;
+        const int steps = (m + 3) / 4;
+        for (int e = m; e < 4 * steps; ++e) t.krow[4 * t.nq + e] = -1;
+        for (int q = 0; q < steps; ++q) t.kcls[t.nq + q] = (signed char)c;
+        t.nq += steps;
+    }
+    t.kfirst[8] = t.nq;
+    return t;
+}
+// 16-row blocks of an S-row operator and the bound that keeps an operator
+// chunk's fragments within LDS (k steps of a chunk <= 60 / row blocks).
 AFMM_HD constexpr int m2l_rb(int S) { return (S + 15) / 16; }
 AFMM_HD constexpr int m2l_kb(int S) { return (S + 3) / 4; }
-AFMM_HD constexpr int m2l_kcmax(int S) { return 60 / m2l_rb(S) > 0 ? 60 / m2l_rb(S) : 1; }
-AFMM_HD constexpr int m2l_nkc(int S) { return (m2l_kb(S) + m2l_kcmax(S) - 1) / m2l_kcmax(S); }
-AFMM_HD constexpr int m2l_kc(int S) { return (m2l_kb(S) + m2l_nkc(S) - 1) / m2l_nkc(S); }
-AFMM_HD constexpr int m2l_chunk(int S) { return m2l_rb(S) * m2l_kc(S) * 64; }
 
 // M2L operator tiling (FP64 and split-FP32 MFMA). When S leaves 1-4 rows past
 // a multiple of 16 (p = 5, 6, 8, 9, ...), those tail rows run on the VALU

@@ -149,19 +149,19 @@ Tables build(int p) {
 
 }  // namespace
 
-std::vector<double> mfma_a_layout(const std::vector<double>& cm, int S, int nmat) {
-    const int RB = m2l_rb(S), NKC = m2l_nkc(S), KC = m2l_kc(S), CH = m2l_chunk(S);
-    std::vector<double> out((size_t)nmat * NKC * CH, 0.0);
-    for (int t = 0; t < nmat; ++t)
-        for (int c = 0; c < NKC; ++c)
-            for (int rb = 0; rb < RB; ++rb)
-                for (int kk = 0; kk < KC; ++kk)
-                    for (int lane = 0; lane < 64; ++lane) {
-                        const int row = 16 * rb + lane % 16, col = 4 * (c * KC + kk) + lane / 16;
-                        if (row < S && col < S)
-                            out[((size_t)t * NKC + c) * CH + ((size_t)rb * KC + kk) * 64 + lane] =
-                                cm[(size_t)t * S * S + (size_t)col * S + row];
-                    }
+std::vector<double> level_a_layout(const std::vector<double>& cm, int p) {
+    const int S = nterms(p);
+    const SymTab t = make_sym_tab(p);
+    std::vector<double> out((size_t)8 * t.rb * t.nq * 64, 0.0);
+    for (int c = 0; c < 8; ++c)
+        for (int b = 0; b < t.rb; ++b)
+            for (int q = 0; q < t.nq; ++q)
+                for (int lane = 0; lane < 64; ++lane) {
+                    const int e = 16 * b + lane % 16, col = t.krow[4 * q + lane / 16];
+                    if (e >= t.cnt[c] || col < 0) continue;
+                    out[(((size_t)c * t.rb + b) * t.nq + q) * 64 + lane] =
+                        cm[(size_t)col * S + t.krow[4 * t.kfirst[c] + e]];
+                }
     return out;
 }
 

@@ -27,12 +27,12 @@ struct Tables {
 // Builds (and caches per p for the life of the process) the tables of order p.
 const Tables& tables_for_order(int p);
 
-// Re-lays S x S column-major matrices for v_mfma_f64_16x16x4_f64 A operands:
-// [matrix][k chunk c][row block rb][k step kk within chunk][lane], value
-// T(row = 16 rb + lane%16, col = 4 (c*KC + kk) + lane/16), zero outside
-// S x S (chunking of afmm_math.h m2l_*). A chunk is contiguous and one
-// fragment is one 512-byte run of 64 lanes.
-std::vector<double> mfma_a_layout(const std::vector<double>& colmajor, int S, int nmat);
+// Re-lays the octant-0 operator of m2m or l2l (the first S x S matrix of
+// `colmajor`) for v_mfma_f64_16x16x4_f64 A operands in the class-major order of
+// SymTab: [row class][16-row block of the class][k step][lane], value
+// T(row = row 16 b + lane%16 of the class, col = row lane/16 of the k step),
+// zero in padding. The other octants' operators are its reflections.
+std::vector<double> level_a_layout(const std::vector<double>& colmajor, int p);
 // M2L operators in the FP64 M2L kernel's chunks: MFMA fragments plus VALU tail rows.
 std::vector<double> m2l_a_layout(const std::vector<double>& colmajor, int S, int nmat);
 

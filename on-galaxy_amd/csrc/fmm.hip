@@ -956,106 +956,217 @@ __global__ void __launch_bounds__(W * 64) k_m2l_bf16(int np, int ntiles, const i
 }
 
 // ---- M2M / L2L on FP64 matrix cores ----------------------------------------------
-// out[t] (+)= sum_o T[o] in[src(o, t)] over the 8 octant operators for 16
-// targets of one level per workgroup of 8 waves: wave o applies octant o's
-// operator (v_mfma_f64_16x16x4_f64, all A fragments and B values of a K-chunk
-// loaded before its MFMAs), and the 8 partial 16 x S tiles are summed in LDS
-// in octant order (deterministic).
-//   MODE 0 (M2M, FmmExpansions3D.hpp:242-265): targets are the level's
-//     non-leaf boxes, src(o, t) = child of t in octant o; overwrites Mhat[t].
-//   MODE 1 (L2L, :307-330): targets are the level's boxes in octant order,
-//     src(o, t) = parent if octant(t) == o (one operator per target); adds
-//     into Lhat[t].
+// Both translate between 16 parents of one level (the level's non-leaf boxes)
+// and their up to 8 children with the octant-0 operator alone: the other
+// octants' operators are its reflections (SymTab). One workgroup of 8 waves
+// per 16 parents and 16-row block b; wave c makes block b of the rows of class c.
+//   M2M (FmmExpansions3D.hpp:242-265): the children's multipoles are
+//     transformed over the octants into W (LDS), row class c takes
+//     W_{c ^ class(k)}[k]; overwrites Mhat[parent].
+//   L2L (:307-330): the products of the parent's local are kept apart by
+//     column class, and their transform over the classes gives all children's
+//     rows; adds into Lhat[child].
+// An absent child adds exact zeros, so no parent's sums depend on its tile.
+// Bound by latency (box chain, gathers, operator loads): most levels have fewer
+// workgroups than the GPU has CUs. A wave makes 24 matrix steps per row block
+// at p = 8 and 73 at p = 16 on loads issued ahead of them; an operator per
+// octant, each wave with all its row blocks, took 105 and 1387 steps per octant
+// (the latter with 128 bytes of spills). All levels, M2M and L2L: 1M bodies at
+// p = 8 184 -> 105 and 201 -> 150 us; 300k at p = 12 2140 -> 159 and 2133 -> 200 us, 120k at
+// p = 16 7386 -> 221 and 6655 -> 214 us.
 constexpr int kLevelWaves = 8;
+constexpr int kLevelPad = 17;  // doubles per LDS row of 16 parents (spreads the banks)
+template <int P>
+__constant__ SymTab kSymTab = make_sym_tab(P);
 
-// Degree of coefficient row r (rows n^2 .. (n+1)^2 - 1 hold degree n).
-constexpr int degree_of(int r) {
-    int n = 0;
-    while ((n + 1) * (n + 1) <= r) ++n;
-    return n;
+// Classes transformed at a time, so that W fits LDS twice per CU.
+constexpr int m2m_group_classes(const SymTab& t) {
+    int rows = 0;
+    for (int c = 0; c < 8; ++c) rows = 4 * (t.kfirst[c + 1] - t.kfirst[c]) > rows ? 4 * (t.kfirst[c + 1] - t.kfirst[c]) : rows;
+    int g = 8;
+    while (g > 1 && g * rows * 8 * kLevelPad * 8 > 72 * 1024) g /= 2;
+    return g;
 }
-// Whether the 16 x 4 operator block (row block rb, k step ks) can be nonzero:
-// M2M takes sources of degree <= the target's, L2L of degree >= the target's.
-template <int S, int MODE>
-constexpr bool level_block_nonzero(int rb, int ks) {
-    const int rlo = 16 * rb, clo = 4 * ks;
-    if (rlo >= S || clo >= S) return false;
-    const int rhi = rlo + 15 < S ? rlo + 15 : S - 1, chi = clo + 3 < S ? clo + 3 : S - 1;
-    return MODE == 0 ? degree_of(clo) <= degree_of(rhi) : degree_of(chi) >= degree_of(rlo);
-}
-
-template <int P, int MODE>
-__global__ void __launch_bounds__(kLevelWaves * 64) k_level_mfma(int n, const int* __restrict__ tgt,
-                                                                const int* __restrict__ child_first,
-                                                                const unsigned char* __restrict__ mask,
-                                                                const int* __restrict__ parent,
-                                                                const int* __restrict__ octant,
-                                                                const double* __restrict__ Tsw,
-                                                                const double* __restrict__ in,
-                                                                double* __restrict__ out) {
-    constexpr int S = nterms(P);
-    constexpr int RB = m2l_rb(S), NKC = m2l_nkc(S), KC = m2l_kc(S), CH = m2l_chunk(S);
-    __shared__ double red[16 * RB * 16];  // [row][target], rows padded to RB*16
-    const int tid = threadIdx.x, o = tid >> 6, lane = tid & 63, j = lane & 15, kq = lane >> 4;
-    const int ti = blockIdx.x * 16 + j;
-    const bool valid = ti < n;
-    const int t = valid ? tgt[ti] : -1;
-    int src = -1;
-    if (valid) {
-        if (MODE == 0) {
-            const unsigned mk = mask[t];
-            if ((mk >> o) & 1u) src = child_first[t] + __popc(mk & ((1u << o) - 1u));
-        } else if (octant[t] == o) {
-            src = parent[t];
-        }
+constexpr int m2m_group_rows(const SymTab& t, int g) {
+    int most = 0;
+    for (int c = 0; c < 8; c += g) {
+        const int r = 4 * (t.kfirst[c + g] - t.kfirst[c]);
+        most = r > most ? r : most;
     }
-    for (int e = tid; e < 16 * RB * 16; e += kLevelWaves * 64) red[e] = 0.0;
-    dbl4 acc[RB];
+    return most;
+}
+
+// In-place Walsh-Hadamard transform over the octant bits.
+__device__ __forceinline__ void octant_transform(double (&v)[8]) {
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) acc[rb] = dbl4{0.0, 0.0, 0.0, 0.0};
-    const bool active = __ballot(src >= 0) != 0ull;
-    if (active) {
-        const double* __restrict__ ms = in + (size_t)(src >= 0 ? src : 0) * S;
-        // structurally zero blocks (a third of them at p = 8) are skipped
+    for (int m = 1; m < 8; m <<= 1)
 #pragma unroll
-        for (int c = 0; c < NKC; ++c) {
-            double bv[KC], av[RB * KC];
-            const double* __restrict__ A = Tsw + ((size_t)o * NKC + c) * CH + lane;
-#pragma unroll
-            for (int e = 0; e < RB * KC; ++e)
-                av[e] = level_block_nonzero<S, MODE>(e / KC, c * KC + e % KC) ? A[e * 64] : 0.0;
-#pragma unroll
-            for (int kk = 0; kk < KC; ++kk) {
-                const int k = 4 * (c * KC + kk) + kq;
-                bv[kk] = (src >= 0 && k < S) ? ms[k] : 0.0;
+        for (int o = 0; o < 8; ++o)
+            if (!(o & m)) {
+                const double a = v[o], b = v[o | m];
+                v[o] = a + b;
+                v[o | m] = a - b;
             }
+}
+
+template <int P>
+__global__ void __launch_bounds__(kLevelWaves * 64) k_m2m(int n, const int* __restrict__ tgt,
+                                                         const int* __restrict__ child_first,
+                                                         const unsigned char* __restrict__ mask,
+                                                         const double* __restrict__ A, double* __restrict__ M) {
+    constexpr int S = nterms(P);
+    constexpr SymTab T = make_sym_tab(P);
+    constexpr int NQ = T.nq, RB = T.rb, G = m2m_group_classes(T), ROWS = m2m_group_rows(T, G);
+    constexpr int NT = kLevelWaves * 64, PER = (16 * ROWS + NT - 1) / NT;
+    __shared__ double W[8][ROWS][kLevelPad];
+    __shared__ int box[16], first[16];
+    __shared__ unsigned kids[16];
+    const int tid = threadIdx.x, c = tid >> 6, lane = tid & 63, j = lane & 15, kq = lane >> 4;
+    const int b = blockIdx.y;
+    // storage index of each of this thread's rows (ahead of the box chain)
+    int kr[8 / G][PER];
 #pragma unroll
-            for (int kk = 0; kk < KC; ++kk)
+    for (int g = 0; g < 8; g += G)
 #pragma unroll
-                for (int rb = 0; rb < RB; ++rb)
-                    if (level_block_nonzero<S, MODE>(rb, c * KC + kk))
-                        acc[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[rb * KC + kk], bv[kk], acc[rb], 0, 0, 0);
+        for (int i = 0; i < PER; ++i) {
+            const int q0 = T.kfirst[g], rows = 4 * (T.kfirst[g + G] - q0), e = tid + NT * i;
+            kr[g / G][i] = e < 16 * rows ? kSymTab<P>.krow[4 * q0 + e % rows] : -1;
         }
-    }
-    // octant-ordered sum of the partial tiles
-    for (int w = 0; w < kLevelWaves; ++w) {
-        __syncthreads();
-        if (w == o && active) {
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) red[(16 * rb + kq + 4 * r) * 16 + j] += acc[rb][r];
-        }
+    if (tid < 16) {
+        const int ti = blockIdx.x * 16 + tid;
+        const int t = ti < n ? tgt[ti] : -1;
+        box[tid] = t;
+        first[tid] = t >= 0 ? child_first[t] : 0;
+        kids[tid] = t >= 0 ? mask[t] : 0u;
     }
     __syncthreads();
-    // write: thread e covers (row, target) pairs
-    for (int e = tid; e < S * 16; e += kLevelWaves * 64) {
-        const int row = e >> 4, jj = e & 15;
-        const int tj = blockIdx.x * 16 + jj;
-        if (tj >= n) continue;
-        const int tt = tgt[tj];
-        if (MODE == 0) out[(size_t)tt * S + row] = red[row * 16 + jj];
-        else out[(size_t)tt * S + row] += red[row * 16 + jj];
+    dbl4 acc{0.0, 0.0, 0.0, 0.0};
+    const double* __restrict__ Ac = A + ((size_t)c * RB + b) * NQ * 64 + lane;
+#pragma unroll
+    for (int g = 0; g < 8; g += G) {
+        const int q0 = T.kfirst[g], rows = 4 * (T.kfirst[g + G] - q0);
+        // the classes' fragments and inputs, all in flight before the transform
+        double a[ROWS / 4];
+#pragma unroll
+        for (int i = 0; i < ROWS / 4; ++i) a[i] = 4 * i < rows ? Ac[(q0 + i) * 64] : 0.0;
+        double v[PER][8];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int e = tid + NT * i, jp = e / rows;
+            const int k = kr[g / G][i];
+            const unsigned mk = k >= 0 ? kids[jp] : 0u;
+            const double* __restrict__ src = M + (size_t)(k >= 0 ? first[jp] : 0) * S + (k >= 0 ? k : 0);
+#pragma unroll
+            for (int o = 0; o < 8; ++o)
+                v[i][o] = (mk >> o) & 1u ? src[(size_t)__popc(mk & ((1u << o) - 1u)) * S] : 0.0;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (the loads stay above)
+        if (g > 0) __syncthreads();  // the previous classes' readers are done
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int e = tid + NT * i, jp = e / rows, row = e - jp * rows;
+            octant_transform(v[i]);
+            if (e < 16 * rows)
+#pragma unroll
+                for (int o = 0; o < 8; ++o) W[o][row][jp] = v[i][o];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ROWS / 4; ++i)
+            if (4 * i < rows)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], W[c ^ T.kcls[q0 + i]][4 * i + kq][j], acc, 0, 0, 0);
+    }
+    const int t = box[j];
+    if (t < 0) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int e = 16 * b + kq + 4 * r;
+        if (e < T.cnt[c]) M[(size_t)t * S + kSymTab<P>.krow[4 * kSymTab<P>.kfirst[c] + e]] = acc[r];
+    }
+}
+
+template <int P>
+__global__ void __launch_bounds__(kLevelWaves * 64) k_l2l(int n, const int* __restrict__ tgt,
+                                                         const int* __restrict__ child_first,
+                                                         const unsigned char* __restrict__ mask,
+                                                         const double* __restrict__ A, double* L) {
+    constexpr int S = nterms(P);
+    constexpr SymTab T = make_sym_tab(P);
+    constexpr int NQ = T.nq, RB = T.rb, NT = kLevelWaves * 64;
+    __shared__ double B[4 * NQ][kLevelPad];
+    __shared__ int box[16];
+    const int tid = threadIdx.x, c = tid >> 6, lane = tid & 63, j = lane & 15, kq = lane >> 4;
+    const int b = blockIdx.y;
+    constexpr int PER = (16 * 4 * NQ + NT - 1) / NT;
+    int kr[PER];  // storage index of each of this thread's rows (ahead of the box chain)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) kr[i] = tid + NT * i < 16 * 4 * NQ ? kSymTab<P>.krow[(tid + NT * i) % (4 * NQ)] : -1;
+    if (tid < 16) box[tid] = (int)blockIdx.x * 16 + tid < n ? tgt[blockIdx.x * 16 + tid] : -1;
+    __syncthreads();
+    double in[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = tid + NT * i, jp = e / (4 * NQ), t = e < 16 * 4 * NQ ? box[jp] : -1;
+        in[i] = t >= 0 && kr[i] >= 0 ? L[(size_t)t * S + kr[i]] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = tid + NT * i, jp = e / (4 * NQ);
+        if (e < 16 * 4 * NQ) B[e - jp * (4 * NQ)][jp] = in[i];
+    }
+    const int t = box[j];
+    const unsigned mk = t >= 0 ? mask[t] : 0u;
+    const int cf = t >= 0 ? child_first[t] : 0;
+    __syncthreads();
+    // the children's values at this lane's four rows, loaded ahead of the products
+    double old[4][8];
+    const double* Lin = L;
+    int row[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int e = 16 * b + kq + 4 * r;
+        row[r] = e < T.cnt[c] ? kSymTab<P>.krow[4 * kSymTab<P>.kfirst[c] + e] : -1;
+#pragma unroll
+        for (int o = 0; o < 8; ++o)
+            old[r][o] = row[r] >= 0 && ((mk >> o) & 1u)
+                            ? Lin[(size_t)(cf + __popc(mk & ((1u << o) - 1u))) * S + row[r]] : 0.0;
+    }
+    // one accumulator per column class
+    dbl4 acc[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) acc[s] = dbl4{0.0, 0.0, 0.0, 0.0};
+    const double* __restrict__ Ac = A + ((size_t)c * RB + b) * NQ * 64 + lane;
+    // (fragments one class ahead of their use)
+    constexpr int KMAX = m2m_group_rows(T, 1) / 4;
+    double a[2][KMAX];
+    auto load_a = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < KMAX; ++i)
+            if (T.kfirst[s] + i < T.kfirst[s + 1]) a[s & 1][i] = Ac[(T.kfirst[s] + i) * 64];
+    };
+    load_a(0);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        if (s < 7) load_a(s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < KMAX; ++i)
+            if (T.kfirst[s] + i < T.kfirst[s + 1])
+                acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s & 1][i], B[4 * (T.kfirst[s] + i) + kq][j], acc[s], 0,
+                                                               0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        double v[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) v[s] = acc[s][r];
+        octant_transform(v);
+        if (row[r] < 0) continue;
+#pragma unroll
+        for (int o = 0; o < 8; ++o)
+            if ((mk >> o) & 1u)
+                L[(size_t)(cf + __popc(mk & ((1u << o) - 1u))) * S + row[r]] =
+                    old[r][o] + ((__popc(o & c) & 1) ? -v[o] : v[o]);
     }
 }
 
@@ -1471,9 +1582,8 @@ void upward(hipStream_t s, const TreeView& t, const TreeMeta& meta, const FmmTab
     for (int l = t.max_level - 1; l >= 0; --l) {
         const int off = meta.nonleaf_off[l], cnt = meta.nonleaf_off[l + 1] - off;
         if (cnt > 0)
-            hipLaunchKernelGGL((k_level_mfma<P, 0>), dim3((cnt + 15) / 16), dim3(kLevelWaves * 64), 0, s, cnt,
-                               t.nonleaf_ids + off,
-                               t.child_first, t.child_mask, t.parent, t.octant, tab.m2m_sw, M, M);
+            hipLaunchKernelGGL(k_m2m<P>, dim3((cnt + 15) / 16, make_sym_tab(P).rb), dim3(kLevelWaves * 64), 0, s, cnt,
+                               t.nonleaf_ids + off, t.child_first, t.child_mask, tab.m2m_sw, M);
     }
     if (e1) AFMM_CHECK(hipEventRecord(e1, s));
 }
@@ -1617,11 +1727,11 @@ void run(Pool& pool, hipStream_t s, const TreeView& t, const TreeMeta& meta, con
     } else if (t.n_x > 0) {
         hipLaunchKernelGGL((k_accumulate<P, 1>), dim3(xcd_chunk_grid(nb)), dim3(64), 0, s, t, L);
     }
-    for (int l = 1; l <= t.max_level; ++l) {
-        const int off = meta.level_off[l], cnt = meta.level_off[l + 1] - off;
-        hipLaunchKernelGGL((k_level_mfma<P, 1>), dim3((cnt + 15) / 16), dim3(kLevelWaves * 64), 0, s, cnt,
-                           t.lo_order + off,
-                           t.child_first, t.child_mask, t.parent, t.octant, tab.l2l_sw, L, L);
+    for (int l = 0; l < t.max_level; ++l) {
+        const int off = meta.nonleaf_off[l], cnt = meta.nonleaf_off[l + 1] - off;
+        if (cnt > 0)
+            hipLaunchKernelGGL(k_l2l<P>, dim3((cnt + 15) / 16, make_sym_tab(P).rb), dim3(kLevelWaves * 64), 0, s, cnt,
+                               t.nonleaf_ids + off, t.child_first, t.child_mask, tab.l2l_sw, L);
     }
     if (ev) AFMM_CHECK(hipEventRecord(ev[3], s));
     if (fb) AFMM_CHECK(hipStreamWaitEvent(s, side.w_done, 0));
