@@ -301,11 +301,12 @@ int afmm_set_graph(afmm_ctx* ctx, int enable);
  * schedule also leave the results' bits unchanged, while the P2P lane grouping
  * changes the order of each near-field sum (same accuracy, different last bits). */
 typedef struct {
-    int32_t m2l_waves;        /* waves per M2L workgroup: 8 or 16. One wave per 16 targets, except
-                                 16 waves of the FP64 M2L above p = 8 and of the split-FP32 M2L,
-                                 where two waves share 16 targets (half the row blocks each).
-                                 Default 16 for FP64 at p <= 8 and p >= 14 and for bf16 at p <= 7,
-                                 else 8 */
+    int32_t m2l_waves;        /* width of the M2L workgroups: 8 or 16. The mixed forms: waves per
+                                 workgroup, one per 16 targets, except 16 waves of the split-FP32
+                                 M2L, where two waves share 16 targets. FP64 (8 waves in either case):
+                                 at p = 7 and 8 tiles of up to 256 (16) or 128 (8) targets, no effect
+                                 at other orders. Default 16 for FP64 at p <= 8 and p >= 14 and for
+                                 bf16 at p <= 7, else 8 */
     int32_t p2p_pair_bodies;  /* leaves with more bodies give each P2P lane two targets (default 32) */
     int32_t p2p_min_group;    /* fewest lanes sharing one target's sources: 1, 2, 4, ..., 64 (default 8) */
     int32_t p2p_schedule;     /* 1: persistent workgroups over the leaves sorted by work bin, largest

@@ -128,7 +128,7 @@ int afmm::eval_forest(afmm_ctx* c, int nsys, const int* sys_off, const double* G
     auto on_core = [&](const TreeView& t, const TreeMeta& m) {
         AFMM_CHECK(hipEventRecord(c->up_fork, s));
         AFMM_CHECK(hipStreamWaitEvent(c->side, c->up_fork, 0));
-        run_upward(c->pool, c->side, t, m, c->prm.p, tab, c->ev[2], c->ev[3]);
+        run_upward(c->pool, c->side, t, m, c->prm.p, c->prm.precision, tab, c->ev[2], c->ev[3]);
         AFMM_CHECK(hipEventRecord(c->up_done, c->side));
         up_launched = true;
     };
@@ -136,7 +136,7 @@ int afmm::eval_forest(afmm_ctx* c, int nsys, const int* sys_off, const double* G
     // the U, W and X lists that M2L does not need.
     bool prep_done = false, m2l_launched = false;
     auto on_vlists = [&](const TreeView& t, const TreeMeta&) {
-        run_m2l_prep(c->pool, s, t, c->prm.p, c->prm.precision, c->shapes);
+        run_m2l_prep(c->pool, s, t, c->prm.p, c->prm.precision);
         prep_done = true;
         if (lists_beside) {
             AFMM_CHECK(hipStreamWaitEvent(s, c->up_done, 0));  // the multipoles are done
@@ -147,7 +147,8 @@ int afmm::eval_forest(afmm_ctx* c, int nsys, const int* sys_off, const double* G
     };
     build_forest(c->pool, s, pos, mass, nsys, sys_off, eps, c->prm.leaf_cap, tv, meta, roots,
                  split ? TreeHook(on_core) : TreeHook(), split ? TreeHook(on_vlists) : TreeHook(),
-                 lists_beside ? c->side : nullptr, c->list_fork, &c->key_levels_hint, &c->tree_depth_hint);
+                 lists_beside ? c->side : nullptr, c->list_fork, &c->key_levels_hint, &c->tree_depth_hint,
+                 m2l_tile_rule(c->prm.p, c->prm.precision, c->shapes.m2l_waves));
     for (const RootInfo& r : roots)
         if (r.nonfinite) return fail(c, AFMM_ERR_NONFINITE, "position or mass is NaN or Inf");
     if (lists_beside) {
@@ -326,20 +327,25 @@ int afmm_create(const afmm_params* prm, afmm_ctx** out) {
         const Tables& T = tables_for_order(prm->p);
         const std::vector<double> m2m = level_a_layout(T.m2m, prm->p);
         const std::vector<double> l2l = level_a_layout(T.l2l, prm->p);
-        // M2L operators in slot order (the order the M2L kernels step through them)
+        c->d_m2m_sw = c->pool.get<double>("T_m2m_sw", m2m.size());
+        c->d_l2l_sw = c->pool.get<double>("T_l2l_sw", l2l.size());
+        AFMM_CHECK(hipMemcpy(c->d_m2m_sw, m2m.data(), sizeof(double) * m2m.size(), hipMemcpyHostToDevice));
+        AFMM_CHECK(hipMemcpy(c->d_l2l_sw, l2l.data(), sizeof(double) * l2l.size(), hipMemcpyHostToDevice));
+        const int form = m2l_form(prm->precision);
+        if (form == kPrecFP64) {
+            const std::vector<double> m2l = m2l_sym_layout(T.m2l, prm->p);
+            c->d_m2l_sw = c->pool.get<double>("T_m2l_sw", m2l.size());
+            AFMM_CHECK(hipMemcpy(c->d_m2l_sw, m2l.data(), sizeof(double) * m2l.size(), hipMemcpyHostToDevice));
+            return AFMM_OK;
+        }
+        // M2L operators in slot order (the order the mixed-precision kernels step through them)
         std::vector<double> m2l_slots(T.m2l.size());
         const size_t SS = (size_t)T.S * T.S;
         for (int k = 0; k < kNumOffsets; ++k)
             std::copy(T.m2l.begin() + kM2LSlotsHost.offset_of[k] * SS,
                       T.m2l.begin() + (kM2LSlotsHost.offset_of[k] + 1) * SS, m2l_slots.begin() + k * SS);
-        const std::vector<double> m2l = m2l_a_layout(m2l_slots, T.S, kNumOffsets);
-        c->d_m2m_sw = c->pool.get<double>("T_m2m_sw", m2m.size());
-        c->d_l2l_sw = c->pool.get<double>("T_l2l_sw", l2l.size());
-        c->d_m2l_sw = c->pool.get<double>("T_m2l_sw", m2l.size());
-        AFMM_CHECK(hipMemcpy(c->d_m2m_sw, m2m.data(), sizeof(double) * m2m.size(), hipMemcpyHostToDevice));
-        AFMM_CHECK(hipMemcpy(c->d_l2l_sw, l2l.data(), sizeof(double) * l2l.size(), hipMemcpyHostToDevice));
-        AFMM_CHECK(hipMemcpy(c->d_m2l_sw, m2l.data(), sizeof(double) * m2l.size(), hipMemcpyHostToDevice));
-        if (m2l_form(prm->precision) == kPrecMixed) {
+        if (form == kPrecMixed) {
+            const std::vector<double> m2l = m2l_a_layout(m2l_slots, T.S, kNumOffsets);
             std::vector<float2> hl(m2l.size());
             for (size_t i = 0; i < m2l.size(); ++i) {
                 const float hi = (float)m2l[i];
@@ -347,8 +353,7 @@ int afmm_create(const afmm_params* prm, afmm_ctx** out) {
             }
             c->d_m2l_hl = c->pool.get<float2>("T_m2l_hl", hl.size());
             AFMM_CHECK(hipMemcpy(c->d_m2l_hl, hl.data(), sizeof(float2) * hl.size(), hipMemcpyHostToDevice));
-        }
-        if (m2l_form(prm->precision) == kPrecMixedBf16) {
+        } else {
             const std::vector<uint16_t> bf = mfma_bf16_layout(m2l_slots, T.S, kNumOffsets);
             c->d_m2l_bf = c->pool.get<uint4>("T_m2l_bf", bf.size() / 8);
             AFMM_CHECK(hipMemcpy(c->d_m2l_bf, bf.data(), sizeof(uint16_t) * bf.size(), hipMemcpyHostToDevice));

@@ -11,8 +11,9 @@
 //              seg_first/seg_count index the sorted bodies.
 //   lists      colleague (27 slots/box) and V (189 slots/box); U, W (per
 //              leaf) and X (per box) in CSR. M2L builds its own transposed
-//              source table srcT[343][targets in (level, octant) order].
-//   expansions Mhat[B][S], Lhat[B][S] (FP64, scaled real basis).
+//              source table srcT[216][targets in (octant, level) order].
+//   expansions Mhat[B][S], Lhat[B][S] (FP64, scaled real basis); the FP64 M2L
+//              reads a copy of Mhat packed in its column order.
 // ============================================================================
 #pragma once
 
@@ -141,13 +142,9 @@ struct TreeView {
     int* lo_order;       // [B] boxes sorted by (level, octant); level l is [level_off[l], level_off[l+1])
     int* m2l_order;      // [B] boxes sorted by (octant, level): the M2L target order
     // M2L target tiles over m2l_order, cut inside octant groups: tile k is
-    // ranks [m2l_tiles{256,128}[k], [k+1]), for workgroups of at most 256
-    // (128) targets; below a CU's worth of full tiles, tiles are cut smaller
-    // (a multiple of 64 targets, or 16 or 32 for the 256 plan) so that they
-    // spread over more CUs
-    int *m2l_tiles256, *m2l_tiles128;
-    int m2l_ntiles256 = 0, m2l_ntiles128 = 0;
-    int m2l_t256 = 256;  // targets per tile of the 256 plan (16 and 32: row-split workgroups)
+    // ranks [m2l_tiles[k], [k+1]), of at most m2l_tile targets (M2LTileRule)
+    int* m2l_tiles;
+    int m2l_ntiles = 0, m2l_tile = 0;
     int* nonleaf_ids;    // [B - nleaves] non-leaf boxes in BFS order
     // lists
     int *coll, *ncoll;   // [27B], [B]
@@ -217,12 +214,23 @@ int radix_sort(SortBufs& b, int n, int first_digit, int ndigits, hipStream_t s, 
 // deepest level, taken as a guess of the levels the key sort must order
 // (verified by the topology passes, all levels sorted again if too shallow);
 // set to this tree's deepest level.
+// tiles: the sizes an M2L tile may have.
+// The M2L tile sizes of an order, precision and workgroup shape: at most
+// `most` targets, and below a CU's worth of such tiles the smallest size whose
+// tiles still fit one per CU: multiples of 64 (one 16-target column block per
+// SIMD) and, with `small` (the FP64 form, whose waves share a column block's
+// rows, and 16-wave workgroups), also 16 and 32.
+struct M2LTileRule {
+    int most;
+    bool small;
+    int per_cu;  // workgroups of 64 and more targets that share a CU
+};
 using TreeHook = std::function<void(const TreeView&, const TreeMeta&)>;
 void build_forest(Pool& pool, hipStream_t s, const double* d_pos, const double* d_mass, int nsys,
                   const int* h_sys_off, const double* h_eps_floor, int cap, TreeView& tv, TreeMeta& meta,
                   std::vector<RootInfo>& roots, const TreeHook& on_core = {}, const TreeHook& on_vlists = {},
                   hipStream_t ls = nullptr, hipEvent_t ls_ready = nullptr, int* levels_hint = nullptr,
-                  int* depth_hint = nullptr);
+                  int* depth_hint = nullptr, M2LTileRule tiles = M2LTileRule{256, false, 1});
 
 // ---- fmm.hip -----------------------------------------------------------------
 struct FmmTimes {
@@ -230,8 +238,8 @@ struct FmmTimes {
 };
 struct FmmTables {
     const double *m2m_sw, *l2l_sw;  // device, octant-0 operators in class-major MFMA A fragments (level_a_layout)
-    const double* m2l_sw;           // device, 343 offset operators in MFMA A fragments (m2l_a_layout)
-    const float2* m2l_hl;           // device, the same as FP32 (hi, lo) pairs, or null
+    const double* m2l_sw;           // device, the FP64 M2L's slot operators (m2l_sym_layout), or null
+    const float2* m2l_hl;           // device, 343 offset operators as FP32 (hi, lo) pairs (m2l_a_layout), or null
     const uint4* m2l_bf;            // device, three-piece bf16 layout (mfma_bf16_layout), or null
 };
 // precision of an evaluation (the values of AFMM_PRECISION_*)
@@ -279,8 +287,8 @@ struct SideStream {
 };
 // The M2L preparation alone on stream s (needs the V lists and the M2L order);
 // a run_fmm with side.prep_done then skips it.
-// Kernel shapes (afmm_shapes of afmm.h with the defaults resolved): waves per
-// M2L workgroup (16 targets each), the leaf size above which a P2P lane takes
+// Kernel shapes (afmm_shapes of afmm.h with the defaults resolved): width of the
+// M2L workgroups, the leaf size above which a P2P lane takes
 // two targets, the fewest lanes per P2P target, and the P2P schedule (0: leaves
 // in XCD chunks in tree order; 1: persistent workgroups over the leaves sorted
 // by work bin, largest first).
@@ -290,24 +298,36 @@ struct Shapes {
     int p2p_min_group = 8;
     int p2p_schedule = 0;
 };
-// The default M2L workgroup of order p and precision mode prec, from
-// measurements on the 1M merger: FP64 16 waves up to p = 8 (one wave per
-// 16-target block) and from p = 14 (two waves per block, half the row blocks
-// each: p = 14 48.8 -> 41.9 ms, p = 16 78.7 -> 73.8 ms per evaluation, where
-// 8 waves spilled), 8 waves at p = 9..13 (p = 10 and 12 8% and 1% faster than
-// the 16-wave split); split FP32 8 waves (7.6 against 8.5 ms at p = 8); the
-// bf16 form 16 waves up to p = 7, 8 above (its FP64 fold totals).
+// The default M2L width of order p and precision mode prec (measured on the 1M
+// merger): split FP32 8 waves (7.6 against 8.5 ms at p = 8); the bf16 form 16
+// waves up to p = 7, 8 above (its FP64 fold totals); FP64 tiles of 256 targets
+// at p = 7 and 8 (no effect at other orders).
 inline int default_m2l_waves(int p, int prec) {
     const int form = m2l_form(prec);
     if (form == kPrecMixedBf16) return p <= 7 ? 16 : 8;
     if (form == kPrecMixed) return 8;
     return p <= 8 || p >= 14 ? 16 : 8;
 }
-void run_m2l_prep(Pool& pool, hipStream_t s, const TreeView& tv, int p, int prec, const Shapes& sh);
+// ---- m2l_fp64.hip --------------------------------------------------------------
+// The FP64 M2L of np targets in the M2L order, cut into ntiles tiles of at most
+// `tile` targets: L[target] = sum over its V list, from packed multipoles Mp
+// (row np all zeros), the slot operators A (m2l_sym_layout), the source table
+// srcT and the tiles' slot presence.
+struct M2LArgs {
+    int np, ntiles, tile;
+    const int *tstart, *order, *ic, *srcT, *present;
+    const double *A, *Mp;
+    double* L;
+};
+void m2l_fp64(hipStream_t s, int p, const M2LArgs& a);
+// The tile sizes of order p, precision prec and shape m2l_waves.
+M2LTileRule m2l_tile_rule(int p, int prec, int waves);
+
+void run_m2l_prep(Pool& pool, hipStream_t s, const TreeView& tv, int p, int prec);
 // P2M and M2M alone on stream s (events e0/e1 around them when non-null); a
 // run_fmm with side.upward_launched then skips them.
-void run_upward(Pool& pool, hipStream_t s, const TreeView& tv, const TreeMeta& meta, int p, const FmmTables& tab,
-                hipEvent_t e0, hipEvent_t e1);
+void run_upward(Pool& pool, hipStream_t s, const TreeView& tv, const TreeMeta& meta, int p, int prec,
+                const FmmTables& tab, hipEvent_t e0, hipEvent_t e1);
 // M2L alone on stream s, after the M2L preparation (the split of the
 // multipoles into bf16 planes included); events e0/e1 around it when non-null.
 void run_m2l(Pool& pool, hipStream_t s, const TreeView& tv, int p, const FmmTables& tab, int prec, const Shapes& sh,

@@ -352,6 +352,136 @@ constexpr SymTab make_sym_tab(int p) {
 AFMM_HD constexpr int m2l_rb(int S) { return (S + 15) / 16; }
 AFMM_HD constexpr int m2l_kb(int S) { return (S + 3) / 4; }
 
+// ---- FP64 M2L plan -----------------------------------------------------------------
+// Sources of one target at mirrored offsets share one operator: with NX axes
+// reflected (the last NX of x, y, z) a slot is an offset with non-negative
+// components on those axes, its up to 2^NX mirror images are transformed into
+// 2^NX combinations, and row class i takes combination i ^ class(k) at column k
+// (SymTab with the classes of the reflected axes). A target meets 189 offsets
+// but only 84 slots at NX = 2 and 56 at NX = 3, an S x S product each.
+// Columns: class-major k steps of 4 (krow, kcls), taken in pairs; a packed
+// multipole stores coefficient (step q, k e) at 8 (q / 2) + 2 e + q % 2, so that
+// 16 bytes hold one k of both steps of a pair. Rows: 16-row blocks per class
+// (v_mfma_f64_16x16x4) and its remainder of at most 12 rows in quads of 4
+// (v_mfma_f64_4x4x4, a quarter of the time).
+constexpr int m2l_axes(int p) { return p >= 4 ? 2 : 1; }
+constexpr int kPlanSteps = kMaxTerms / 4 + 8, kPlanBlocks = 24, kPlanQuads = 24;
+struct M2LPlan {
+    int nq = 0, nb = 0, nd = 0;           // k steps, row blocks, quads
+    int npad = 0;                         // unused positions of a packed multipole
+    short krow[4 * kPlanSteps] = {};      // storage index (-1: padding)
+    signed char kcls[kPlanSteps] = {};
+    short brow[16 * kPlanBlocks] = {};    // storage index of each block row (-1: padding)
+    signed char bcls[kPlanBlocks] = {};
+    short drow[4 * kPlanQuads] = {};      // ... of each quad row
+    signed char dcls[kPlanQuads] = {};
+    short kpos[kMaxTerms] = {};           // packed position of a storage index
+    short pads[64] = {};
+};
+constexpr M2LPlan make_m2l_plan(int p) {
+    M2LPlan t{};
+    const int nx = m2l_axes(p);
+    for (int c = 0; c < (1 << nx); ++c) {
+        short rows[kMaxTerms] = {};
+        int m = 0;
+        for (int n = 0; n <= p; ++n)
+            for (int a = 0; a <= n; ++a)
+                for (int im = 0; im < (a ? 2 : 1); ++im)
+                    if ((sym_class(n, a, im) >> (3 - nx)) == c) rows[m++] = (short)(rid(n, a) + im);
+        const int steps = (m + 3) / 4;
+        for (int e = 0; e < 4 * steps; ++e) {
+            t.krow[4 * t.nq + e] = e < m ? rows[e] : (short)-1;
+            const int q = t.nq + e / 4, pos = 8 * (q / 2) + 2 * (e % 4) + q % 2;
+            if (e < m) t.kpos[rows[e]] = (short)pos;
+            else t.pads[t.npad++] = (short)pos;
+        }
+        for (int q = 0; q < steps; ++q) t.kcls[t.nq + q] = (signed char)c;
+        t.nq += steps;
+        int done = 0;
+        while (done < m) {
+            const bool quad = m - done <= 12;
+            for (int e = 0; e < (quad ? 4 : 16); ++e)
+                (quad ? t.drow[4 * t.nd + e] : t.brow[16 * t.nb + e]) = done + e < m ? rows[done + e] : (short)-1;
+            if (quad) t.dcls[t.nd++] = (signed char)c;
+            else t.bcls[t.nb++] = (signed char)c;
+            done += quad ? 4 : 16;
+        }
+    }
+    if (t.nq % 2)  // the missing step of the last pair
+        for (int e = 0; e < 4; ++e) t.pads[t.npad++] = (short)(8 * (t.nq / 2) + 2 * e + 1);
+    return t;
+}
+// Doubles of a packed multipole, and of one k step of a slot's operator: the
+// blocks' fragments ([block][k][row]), then the quads' ([quad][k][row]).
+constexpr int m2l_pack(int p) { return 8 * ((make_m2l_plan(p).nq + 1) / 2); }
+constexpr int m2l_step(int p) { return make_m2l_plan(p).nb * 64 + make_m2l_plan(p).nd * 16; }
+
+// Workgroups that share a CU: two where two double-buffered operators fit its
+// LDS. Else one, whose waves own two 16-target columns where their accumulators
+// fit the registers.
+constexpr int m2l_workgroups(int p) { return p <= 6 ? 2 : 1; }
+constexpr int m2l_columns(int p) { return p == 7 || p == 8 ? 2 : 1; }
+
+// The slots in the order an M2L workgroup steps through them: offsets of one
+// parity class (mod 2) reach the same lattice of sources, so slots run class by
+// class, inside a class along a boustrophedon path (consecutive slots' sources
+// are mostly the same boxes shifted by one lattice step and stay in the L2).
+// first[k]: the slot's offset_index. row[par][k][m]: the source-table row of its
+// mirror image m (bits of the reflected axes) for a target of parities par (4 x
+// + 2 y + z bits of its coordinates), kSrcRows where the target cannot meet it
+// or it coincides with another image.
+constexpr int kSrcRows = 216;
+constexpr int src_row_of(int dx, int dy, int dz, int par) {
+    const int ux = dx + 3 - (par >> 2), uy = dy + 3 - ((par >> 1) & 1), uz = dz + 3 - (par & 1);
+    return ux >= 0 && ux < 6 && uy >= 0 && uy < 6 && uz >= 0 && uz < 6 ? (ux * 6 + uy) * 6 + uz : kSrcRows;
+}
+template <int NX>
+struct M2LSymSlots {
+    static constexpr int kMost = NX == 3 ? 56 : NX == 2 ? 100 : 178;
+    int n = 0;
+    short first[kMost] = {};
+    short row[8][kMost][1 << NX] = {};
+};
+template <int NX>
+constexpr M2LSymSlots<NX> make_m2l_sym_slots() {
+    constexpr int nx = NX;
+    M2LSymSlots<NX> t{};
+    for (int cls = 0; cls < 8; ++cls) {
+        int vals[3][4] = {}, nv[3] = {0, 0, 0};
+        for (int a = 0; a < 3; ++a)
+            for (int d = a >= 3 - nx ? 0 : -3; d <= 3; ++d)
+                if (((d + 4) & 1) == ((cls >> (2 - a)) & 1)) vals[a][nv[a]++] = d;
+        int line = 0;
+        for (int ix = 0; ix < nv[0]; ++ix)
+            for (int j = 0; j < nv[1]; ++j) {
+                const int iy = (ix & 1) ? nv[1] - 1 - j : j;
+                for (int l = 0; l < nv[2]; ++l) {
+                    const int iz = (line & 1) ? nv[2] - 1 - l : l;
+                    const int d[3] = {vals[0][ix], vals[1][iy], vals[2][iz]};
+                    bool adjacent = true;
+                    for (int a = 0; a < 3; ++a) adjacent = adjacent && d[a] >= -1 && d[a] <= 1;
+                    if (adjacent) continue;
+                    t.first[t.n] = (short)offset_index(d[0], d[1], d[2]);
+                    for (int m = 0; m < (1 << nx); ++m) {
+                        bool own = true;
+                        int v[3] = {d[0], d[1], d[2]};
+                        for (int b = 0; b < nx; ++b)
+                            if ((m >> b) & 1) {
+                                const int a = 3 - nx + b;
+                                own = own && v[a] != 0;
+                                v[a] = -v[a];
+                            }
+                        for (int par = 0; par < 8; ++par)
+                            t.row[par][t.n][m] = own ? (short)src_row_of(v[0], v[1], v[2], par) : (short)kSrcRows;
+                    }
+                    ++t.n;
+                }
+                ++line;
+            }
+    }
+    return t;
+}
+
 // M2L operator tiling (FP64 and split-FP32 MFMA). When S leaves 1-4 rows past
 // a multiple of 16 (p = 5, 6, 8, 9, ...), those tail rows run on the VALU
 // instead of a 16-row MFMA block that would be mostly padding: MRB row blocks

@@ -165,6 +165,36 @@ std::vector<double> level_a_layout(const std::vector<double>& cm, int p) {
     return out;
 }
 
+namespace {
+template <int NX>
+std::vector<double> sym_layout(const std::vector<double>& cm, int p) {
+    constexpr M2LSymSlots<NX> slots = make_m2l_sym_slots<NX>();
+    const int S = nterms(p);
+    const M2LPlan t = make_m2l_plan(p);
+    std::vector<double> out((size_t)slots.n * t.nq * m2l_step(p), 0.0);
+    double* u = out.data();
+    for (int s = 0; s < slots.n; ++s) {
+        const double* T = cm.data() + (size_t)slots.first[s] * S * S;
+        auto at = [&](int row, int col) { return row >= 0 && col >= 0 ? T[(size_t)col * S + row] : 0.0; };
+        for (int q = 0; q < t.nq; ++q) {
+            for (int b = 0; b < t.nb; ++b)
+                for (int lane = 0; lane < 64; ++lane) *u++ = at(t.brow[16 * b + lane % 16], t.krow[4 * q + lane / 16]);
+            for (int d = 0; d < t.nd; ++d)
+                for (int e = 0; e < 16; ++e) *u++ = at(t.drow[4 * d + e % 4], t.krow[4 * q + e / 4]);
+        }
+    }
+    return out;
+}
+}  // namespace
+
+std::vector<double> m2l_sym_layout(const std::vector<double>& cm, int p) {
+    switch (m2l_axes(p)) {
+        case 1: return sym_layout<1>(cm, p);
+        case 2: return sym_layout<2>(cm, p);
+        default: return sym_layout<3>(cm, p);
+    }
+}
+
 std::vector<double> m2l_a_layout(const std::vector<double>& cm, int S, int nmat) {
     const int MRB = m2l_mrb(S), TR = m2l_tail(S), NKC = m2l_mnkc(S), KC = m2l_mkc(S), CH = m2l_mchunk(S);
     std::vector<double> out((size_t)nmat * NKC * CH, 0.0);

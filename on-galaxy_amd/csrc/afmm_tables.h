@@ -33,7 +33,11 @@ const Tables& tables_for_order(int p);
 // T(row = row 16 b + lane%16 of the class, col = row lane/16 of the k step),
 // zero in padding. The other octants' operators are its reflections.
 std::vector<double> level_a_layout(const std::vector<double>& colmajor, int p);
-// M2L operators in the FP64 M2L kernel's chunks: MFMA fragments plus VALU tail rows.
+// The FP64 M2L operators of the slots (M2LPlan, make_m2l_sym_slots): [slot][k
+// step][16-row block | quad: k, row] of the slot's offset with
+// non-negative reflected components.
+std::vector<double> m2l_sym_layout(const std::vector<double>& colmajor, int p);
+// M2L operators in the split-FP32 M2L kernel's chunks: MFMA fragments plus VALU tail rows.
 std::vector<double> m2l_a_layout(const std::vector<double>& colmajor, int S, int nmat);
 
 // The same matrices for v_mfma_f32_16x16x32_bf16, each entry split into three

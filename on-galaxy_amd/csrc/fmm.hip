@@ -11,8 +11,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "afmm_internal.h"
-#include "afmm_math.h"
+#include "m2l_common.h"
 
 namespace afmm {
 namespace {
@@ -20,20 +19,10 @@ namespace {
 constexpr int kT = 256;
 inline int blocks(long long n, int t = kT) { return (int)std::max<long long>(1, (n + t - 1) / t); }
 
-// ---- XCD-aware workgroup order ------------------------------------------------
-// MI355X deals workgroups round-robin to its 8 XCDs, each with its own L2.
-// Kernels whose neighbouring work items (tiles or leaves in tree order) read
-// the same neighbour data launch xcd_grid(n) workgroups and take item
-// xcd_item(): each XCD then runs one contiguous range of items, in order, and
-// the shared reads hit its L2. Items >= n return at once.
+// ---- XCD-aware workgroup order in chunks (xcd_item: m2l_common.h) --------------
 // Per-leaf kernels, whose cost varies from leaf to leaf in spatial clusters,
 // use chunks of K items instead (xcd_chunk_*): chunks go round-robin to the
 // XCDs, which keeps each XCD's share balanced and its reads local within a chunk.
-constexpr int kXcds = 8;
-inline int xcd_grid(int n) { return (n + kXcds - 1) / kXcds * kXcds; }
-__device__ __forceinline__ int xcd_item() {
-    return (int)(blockIdx.x % kXcds) * (int)(gridDim.x / kXcds) + (int)(blockIdx.x / kXcds);
-}
 constexpr int kLeafChunk = 32;
 inline int xcd_chunk_grid(int n) { return (n + kXcds * kLeafChunk - 1) / (kXcds * kLeafChunk) * (kXcds * kLeafChunk); }
 __device__ __forceinline__ int xcd_chunk_item() {
@@ -86,6 +75,10 @@ template <int S>
 constexpr int coef_windows() { return S <= 96 ? 1 : ((S + 127) / 128 > 2 ? (S + 127) / 128 : 2); }
 template <int S>
 constexpr int coef_window() { return (S + coef_windows<S>() - 1) / coef_windows<S>(); }
+
+// Where a coefficient goes in the packed multipoles of the FP64 M2L.
+template <int P>
+__constant__ M2LPlan kPack = make_m2l_plan(P);
 
 // Bodies of a list of boxes staged through LDS in chunks of kStreamChunk list
 // entries: their (first body, count) and the running body offset, so that
@@ -149,7 +142,8 @@ __device__ __forceinline__ int stream_body(const StreamLds& sl, int m, int q) {
 template <int P, int KIND, int C0, int CW>
 __device__ __forceinline__ void accumulate_window(const TreeView& t, const int* list, int nlist, int f0, int n0,
                                                   const double* ch, double ih, int lane, StreamLds& sl,
-                                                  double* __restrict__ out, size_t out_base) {
+                                                  double* __restrict__ out, size_t out_base,
+                                                  double* __restrict__ packed = nullptr) {
     constexpr int S = nterms(P);
     double acc[CW];
 #pragma unroll
@@ -195,13 +189,15 @@ __device__ __forceinline__ void accumulate_window(const TreeView& t, const int* 
         if (k < cnt && C0 + first + k < S) {
             if constexpr (KIND == 1) out[out_base + C0 + first + k] += acc[k];
             else out[out_base + C0 + first + k] = acc[k];
+            if (KIND == 0 && packed) packed[kPack<P>.kpos[C0 + first + k]] = acc[k];
         }
 }
 
 // One wave per box (four waves per box with X lists measured 2.7x slower:
 // most X ranges hold too few bodies to occupy them).
+// Mp (KIND 0, may be null): the packed multipoles of the FP64 M2L, written too.
 template <int P, int KIND>
-__global__ void __launch_bounds__(64) k_accumulate(TreeView t, double* __restrict__ out) {
+__global__ void __launch_bounds__(64) k_accumulate(TreeView t, double* __restrict__ out, double* __restrict__ Mp) {
     constexpr int S = nterms(P);
     constexpr int CW = coef_window<S>();
     __shared__ StreamLds sl;
@@ -226,12 +222,16 @@ __global__ void __launch_bounds__(64) k_accumulate(TreeView t, double* __restric
                           t.cdd[6 * (size_t)b + 3], t.cdd[6 * (size_t)b + 4], t.cdd[6 * (size_t)b + 5]};
     const double ih = t.invh[b];
     const int f0 = KIND == 0 ? t.seg_first[b] : 0, n0 = KIND == 0 ? t.seg_count[b] : 0;
-    accumulate_window<P, KIND, 0, CW>(t, list, nlist, f0, n0, ch, ih, lane, sl, out, (size_t)b * S);
+    constexpr int SP = m2l_pack(P);
+    double* const pk = KIND == 0 && Mp ? Mp + (size_t)b * SP : nullptr;
+    if (pk && lane < kPack<P>.npad) pk[kPack<P>.pads[lane]] = 0.0;
+    accumulate_window<P, KIND, 0, CW>(t, list, nlist, f0, n0, ch, ih, lane, sl, out, (size_t)b * S, pk);
     if constexpr (CW < S)
         accumulate_window<P, KIND, CW, (2 * CW < S ? CW : S - CW)>(t, list, nlist, f0, n0, ch, ih, lane, sl, out,
-                                                                   (size_t)b * S);
+                                                                   (size_t)b * S, pk);
     if constexpr (2 * CW < S)
-        accumulate_window<P, KIND, 2 * CW, S - 2 * CW>(t, list, nlist, f0, n0, ch, ih, lane, sl, out, (size_t)b * S);
+        accumulate_window<P, KIND, 2 * CW, S - 2 * CW>(t, list, nlist, f0, n0, ch, ih, lane, sl, out, (size_t)b * S,
+                                                       pk);
     static_assert(3 * CW >= S, "three coefficient windows cover every order built");
 }
 
@@ -359,8 +359,6 @@ __global__ void __launch_bounds__(kM2PWaves * 64, m2p_min_waves<P>()) k_m2p(Tree
 // j + 16k, D[i][j] in lane j + 16(i%4), register i/4 (rows interleave by 4,
 // unlike the f32 16x16x4 form; see ck's mfma_type for f64 16x16x4:
 // group_size 1, num_groups_per_blk 4).
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-
 __global__ void __launch_bounds__(kT) k_zero_int(int* a, size_t n) {
     const size_t i = blockIdx.x * (size_t)kT + threadIdx.x;
     if (i < n) a[i] = 0;
@@ -370,25 +368,24 @@ __global__ void __launch_bounds__(kT) k_zero_int(int* a, size_t n) {
 // operators are all kept in slot order).
 __constant__ M2LSlots kM2LSlots = make_m2l_slots();
 
-// Source-table rows: a target at integer coordinate 2 P + c (c = 0 or 1 per
-// axis, the parities par = 4 cx + 2 cy + cz) meets its V-list sources, the
-// children of its parent's colleagues P - 1 .. P + 1 that are not adjacent,
-// only at offsets d = ic(target) - ic(source) in [c - 3, c + 2]: 6 of the 7
-// values per axis, 216 of the 343 offsets. Row of offset index oi (of
-// offset_index) for parities par, or -1 where the target cannot meet it.
-constexpr int kSrcRows = 216;
-__device__ __forceinline__ int src_row(int oi, int par) {
-    const int ux = oi / 49 - (par >> 2), uy = (oi / 7) % 7 - ((par >> 1) & 1), uz = oi % 7 - (par & 1);
-    return (unsigned)ux < 6u && (unsigned)uy < 6u && (unsigned)uz < 6u ? (ux * 6 + uy) * 6 + uz : -1;
-}
-__device__ __forceinline__ int ic_parity(const int* __restrict__ ic, int b) {
-    return ((ic[3 * (size_t)b] & 1) << 2) | ((ic[3 * (size_t)b + 1] & 1) << 1) | (ic[3 * (size_t)b + 2] & 1);
+// Slots of the presence table: every offset (NX = -1: the mixed-precision M2L)
+// or the mirrored offsets of the FP64 M2L with NX reflected axes.
+template <int NX>
+__constant__ M2LSymSlots<NX> kSymSlots = make_m2l_sym_slots<NX>();
+template <int NX>
+constexpr int src_slots() {
+    if constexpr (NX < 0) return kNumOffsets;
+    else {
+        constexpr int n = make_m2l_sym_slots<NX>().n;
+        return n;
+    }
 }
 
 // srcT[row * np + r] = the source box of target order[r] at the offset of that
-// row (src_row for the target's parities), -1 where it has none, and
+// row (src_row for the target's parities), -1 (FP64: nb, and a last row of nb) where it has none, and
 // present[tile][slot] = 1 when some target of the tile has a source at that
-// slot (present zeroed before). One block per 16 consecutive targets of the
+// slot (present zeroed before). zero_box (when non-null): a packed multipole of
+// npack values set to zero, which absent sources read. One block per 16 consecutive targets of the
 // M2L order: their V lists fill a rows x 16 table in LDS (initially -1), which
 // is then written out row by row, 64 contiguous bytes per row, so the whole
 // table is written once and coalesced (no separate fill of -1). Presence: one
@@ -396,19 +393,23 @@ __device__ __forceinline__ int ic_parity(const int* __restrict__ ic, int b) {
 // source there (order-free; a block's targets span one tile or a few small
 // ones).
 constexpr int kSrcTargets = 16;
+template <int NX>
 __global__ void __launch_bounds__(kT) k_m2l_src(int nb, int np, const int* __restrict__ order,
                                                const int* __restrict__ vl, const int* __restrict__ nv,
                                                const int* __restrict__ ic, int* __restrict__ srcT,
                                                const int* __restrict__ tstart, int ntiles,
-                                               int* __restrict__ present) {
+                                               int* __restrict__ present, double* __restrict__ zero_box, int npack) {
     __shared__ int tab[kSrcRows][kSrcTargets];
     __shared__ int box[kSrcTargets], cnt[kSrcTargets], tile_of[kSrcTargets], par[kSrcTargets];
     // consecutive blocks on one XCD, so the two 64-byte halves of a 128-byte
     // row segment are written through the same L2
     const int r0 = xcd_item() * kSrcTargets, tid = threadIdx.x;
+    if (NX >= 0 && blockIdx.x == 0)
+        for (int e = tid; e < npack; e += kT) zero_box[e] = 0.0;
     if (r0 >= nb) return;
     const int nt = min(kSrcTargets, nb - r0);
-    for (int e = tid; e < kSrcRows * kSrcTargets; e += kT) (&tab[0][0])[e] = -1;
+    const int none = NX < 0 ? -1 : nb;  // (the FP64 form reads the zero multipole nb)
+    for (int e = tid; e < kSrcRows * kSrcTargets; e += kT) (&tab[0][0])[e] = none;
     if (tid < nt) {
         box[tid] = order[r0 + tid];
         cnt[tid] = nv[box[tid]];
@@ -434,95 +435,65 @@ __global__ void __launch_bounds__(kT) k_m2l_src(int nb, int np, const int* __res
         if (row >= 0) tab[row][j] = c;  // (always: V sources lie in the target's range)
     }
     __syncthreads();
-    for (int e = tid; e < kSrcRows * kSrcTargets; e += kT) {
+    for (int e = tid; e < (kSrcRows + (NX < 0 ? 0 : 1)) * kSrcTargets; e += kT) {
         const int k = e / kSrcTargets, j = e - k * kSrcTargets;
-        if (j < nt) srcT[(size_t)k * np + r0 + j] = tab[k][j];
+        if (j < nt) srcT[(size_t)k * np + r0 + j] = k < kSrcRows ? tab[k][j] : none;
     }
-    for (int k = tid; k < kNumOffsets; k += kT) {
-        const int oi = kM2LSlots.offset_of[k];
+    constexpr int NS = src_slots<NX>();
+    for (int k = tid; k < NS; k += kT) {
         bool any = false;
         for (int j = 0; j < nt; ++j) {
-            const int row = src_row(oi, par[j]);
-            any |= row >= 0 && tab[row][j] >= 0;
+            if constexpr (NX < 0) {
+                const int row = src_row(kM2LSlots.offset_of[k], par[j]);
+                any |= row >= 0 && tab[row][j] != none;
+            } else {
+                for (int m = 0; m < (1 << NX); ++m) {
+                    const int row = kSymSlots<NX>.row[par[j]][k][m];
+                    any |= row < kSrcRows && tab[row][j] != none;
+                }
+            }
             if (j + 1 == nt || tile_of[j + 1] != tile_of[j]) {  // end of a run in one tile
-                if (any) atomicOr(&present[(size_t)tile_of[j] * kNumOffsets + k], 1);
+                if (any) atomicOr(&present[(size_t)tile_of[j] * NS + k], 1);
                 any = false;
             }
         }
     }
 }
 
-// Waves per M2L workgroup (W, a kernel shape the autotuner may choose): 16
-// waves (4 per SIMD share the MFMA pipe and hide each other's LDS and gather
-// latency; at p = 8 measured 8% faster than 8 waves of 32 targets) or 8. A
-// wave owns one 16-target column block, except where one block's
-// accumulators would not fit four waves per SIMD (FP64 above p = 8, split
-// FP32): there 16-wave workgroups give each block two waves (m2l_row_split).
+// Waves per workgroup of the mixed-precision M2L forms (W, a kernel shape the
+// autotuner may choose): 16 or 8. A wave owns one 16-target column block,
+// except where one block's accumulators would not fit four waves per SIMD
+// (split FP32): there 16-wave workgroups give each block two waves.
 // The defaults per order and form are in default_m2l_waves.
-constexpr int kM2LCb = 1;  // 16-target column blocks per wave
-
 typedef float flt4 __attribute__((ext_vector_type(4)));
 
-// Waves per 16-target column block of the FP64 / split-FP32 M2L workgroup:
-// with 16 waves, two share each block (half the row blocks each) where one
-// wave's accumulators would not fit four waves per SIMD (above p = 8, and
-// the split-FP32 form with its FP64 fold totals).
-constexpr int m2l_row_split(int p, bool mix, int waves) { return waves == 16 && (p > 8 || mix) ? 2 : 1; }
-// Targets per M2L workgroup (tile) of order p, precision mode prec and waves
-// per workgroup (the bf16 kernel has no row split).
-inline int m2l_tile_targets(int p, int prec, int waves) {
-    const int form = m2l_form(prec);
-    const int rs = form == kPrecMixedBf16 ? 1 : m2l_row_split(p, form == kPrecMixed, waves);
-    return waves / rs * 16 * kM2LCb;
-}
-
-// Operator fragment and accumulator types. FP64: v_mfma_f64_16x16x4f64 on
-// double operators. Split FP32: each operand x is carried as hi = fl32(x),
-// lo = fl32(x - hi), and a 16x16x4 product is three v_mfma_f32_16x16x4f32
-// (lo*hi + hi*lo + hi*hi) into an FP32 accumulator.
-template <bool MIX>
-struct M2LTypes {
-    using A = double;
-    using Acc = dbl4;
-};
-template <>
-struct M2LTypes<true> {
-    using A = float2;
-    using Acc = flt4;
-};
-
-__device__ __forceinline__ double a_value(double a) { return a; }
-__device__ __forceinline__ double a_value(float2 a) { return (double)a.x + (double)a.y; }
-
-// RSX (0: the default row split of the order and form) lets more waves share a
-// column block when tiles are small (16 or 32 targets): each wave then runs a
-// shorter chain per offset, and every row keeps its accumulation order.
-template <int P, bool MIX, int W, int RSX = 0>
-__global__ void __launch_bounds__(W * 64) k_m2l_mfma(int np, int ntiles, const int* __restrict__ tstart,
-                                                           const int* __restrict__ order,
-                                                           const int* __restrict__ ic,
-                                                           const int* __restrict__ srcT,
-                                                           const int* __restrict__ present_g,
-                                                           const typename M2LTypes<MIX>::A* __restrict__ Asw,
-                                                           const double* __restrict__ M, double* __restrict__ L) {
-    using AT = typename M2LTypes<MIX>::A;
-    using Acc = typename M2LTypes<MIX>::Acc;
+// ---- M2L on FP32 matrix cores with split operands --------------------------------
+// Each operand x is carried as hi = fl32(x), lo = fl32(x - hi), and a 16x16x4
+// product is three v_mfma_f32_16x16x4f32 (lo*hi + hi*lo + hi*hi) into an FP32
+// accumulator. A wave owns 16 targets (the columns) and loops over the offsets
+// present in its tile against the gathered source multipoles (B, zero where a
+// target has no source at that offset); with 16 waves, RS = 2 waves share each
+// 16-target column block, each taking RBH of the RB row blocks (the tail rows
+// go to the last of them). A[i][k] in lane i + 16k, B[k][j] in lane j + 16k,
+// D[i][j] in lane j + 16(i/4), register i%4. The FP64 form is in m2l_fp64.hip.
+template <int P, int W>
+__global__ void __launch_bounds__(W * 64) k_m2l_split(int np, int ntiles, const int* __restrict__ tstart,
+                                                      const int* __restrict__ order, const int* __restrict__ ic,
+                                                      const int* __restrict__ srcT,
+                                                      const int* __restrict__ present_g,
+                                                      const float2* __restrict__ Asw, const double* __restrict__ M,
+                                                      double* __restrict__ L) {
     constexpr int S = nterms(P);
     constexpr int RB = m2l_mrb(S), TR = m2l_tail(S), NKC = m2l_mnkc(S), KC = m2l_mkc(S), CH = m2l_mchunk(S);
-    constexpr int CB = kM2LCb;
-    // RS waves share each 16-target column block, each taking RBH of the RB
-    // row blocks (the tail rows go to the last of them): RS = 2 when a whole
-    // column block's accumulators would not fit four waves per SIMD.
-    constexpr int RS = RSX ? RSX : m2l_row_split(P, MIX, W);
+    constexpr int RS = W == 16 ? 2 : 1;
     constexpr int RBH = (RB + RS - 1) / RS;
-    constexpr int TILE = W / RS * 16 * CB;
     constexpr int NT = W * 64;
     constexpr int PER = (CH + NT - 1) / NT;
     // WHOLE: both buffers hold a whole operator (all NKC chunks), so the
     // workgroup synchronises once per offset; otherwise once per chunk.
-    constexpr bool WHOLE = NKC > 1 && 2 * NKC * CH * (int)sizeof(AT) <= 150 * 1024;
+    constexpr bool WHOLE = NKC > 1 && 2 * NKC * CH * (int)sizeof(float2) <= 150 * 1024;
     constexpr int BUFN = WHOLE ? NKC * CH : CH;
-    __shared__ AT abuf[2][BUFN];
+    __shared__ float2 abuf[2][BUFN];
     __shared__ unsigned char present[kNumOffsets + 1];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int grp = wave / RS, rb0 = (wave % RS) * RBH;  // column block, first row block
@@ -530,40 +501,23 @@ __global__ void __launch_bounds__(W * 64) k_m2l_mfma(int np, int ntiles, const i
     const int j = lane & 15, kq = lane >> 4;
     const int tile = xcd_item();
     if (tile >= ntiles) return;
-    const int base = tstart[tile], end = tstart[tile + 1];  // end - base <= TILE
-    int rank[CB], par[CB];
-    bool valid[CB];
+    const int base = tstart[tile], end = tstart[tile + 1];  // end - base <= 16 W / RS
+    const int rank = base + grp * 16 + j;
+    const bool valid = rank < end;
+    const int par = valid ? ic_parity(ic, order[rank]) : 0;
+    // each offset's products are summed in FP32 from zero and folded into FP64
+    // totals when the offset is done, so FP32 rounding never compounds across
+    // the up to 189 offsets of a target
+    flt4 acc[RBH];
+    dbl4 accd[RBH];
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-        rank[cb] = base + (grp * CB + cb) * 16 + j;
-        valid[cb] = rank[cb] < end;
-        par[cb] = valid[cb] ? ic_parity(ic, order[rank[cb]]) : 0;
-    }
-    Acc acc[CB][RBH];
-    // MIX: each offset's products are summed in FP32 from zero and folded into
-    // FP64 totals when the offset is done, so FP32 rounding never compounds
-    // across the up to 189 offsets of a target.
-    dbl4 accd[MIX ? CB : 1][MIX ? RBH : 1];
+    for (int rb = 0; rb < RBH; ++rb)
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int rb = 0; rb < RBH; ++rb)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[cb][rb][r] = 0;
-    if constexpr (MIX)
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < RBH; ++rb)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) accd[cb][rb][r] = 0.0;
-    (void)TILE;
+        for (int r = 0; r < 4; ++r) acc[rb][r] = 0.f, accd[rb][r] = 0.0;
     // tail rows 16 RB + tr: lane (j, kq) sums its k = kq (mod 4) terms
-    double tacc[CB][TR > 0 ? TR : 1];
+    double tacc[TR > 0 ? TR : 1];
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-        for (int tr = 0; tr < (TR > 0 ? TR : 1); ++tr) tacc[cb][tr] = 0.0;
+    for (int tr = 0; tr < (TR > 0 ? TR : 1); ++tr) tacc[tr] = 0.0;
     {
         for (int t = tid; t < kNumOffsets; t += NT) present[t] = present_g[(size_t)tile * kNumOffsets + t];
         if (tid == 0) present[kNumOffsets] = 1;  // sentinel
@@ -576,34 +530,26 @@ __global__ void __launch_bounds__(W * 64) k_m2l_mfma(int np, int ntiles, const i
         // Software pipeline over (offset o, k chunk c) items: while the MFMAs of
         // the current item run, the next item's operator chunk (global -> regs
         // -> other LDS buffer) and its gathered source multipoles are in flight.
-        auto load_b = [&](const int (&src)[CB], int c, double (&bv)[CB][KC]) {
+        auto load_b = [&](int src, int c, double (&bv)[KC]) {
+            const double* ms = M + (size_t)(src >= 0 ? src : 0) * S;
 #pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-                const double* ms = M + (size_t)(src[cb] >= 0 ? src[cb] : 0) * S;
-#pragma unroll
-                for (int kk = 0; kk < KC; ++kk) {
-                    const int k = 4 * (c * KC + kk) + kq;
-                    bv[cb][kk] = (src[cb] >= 0 && k < S) ? ms[k] : 0.0;
-                }
+            for (int kk = 0; kk < KC; ++kk) {
+                const int k = 4 * (c * KC + kk) + kq;
+                bv[kk] = (src >= 0 && k < S) ? ms[k] : 0.0;
             }
         };
-        auto load_src = [&](int o, int (&src)[CB]) {
-            bool any = false;
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-                const int row = o < kNumOffsets && valid[cb] ? src_row(kM2LSlots.offset_of[o], par[cb]) : -1;
-                src[cb] = row >= 0 ? srcT[(size_t)row * np + rank[cb]] : -1;
-                any |= src[cb] >= 0;
-            }
-            return __ballot(any) != 0ull;
+        auto load_src = [&](int o, int& src) {
+            const int row = o < kNumOffsets && valid ? src_row(kM2LSlots.offset_of[o], par) : -1;
+            src = row >= 0 ? srcT[(size_t)row * np + rank] : -1;
+            return __ballot(src >= 0) != 0ull;
         };
         int o = next_present(-1);
-        int scur[CB], snext[CB];
-        double bcur[CB][KC], bnext[CB][KC];
+        int scur = -1, snext = -1;
+        double bcur[KC], bnext[KC];
         bool has_cur = false, has_next = false;
         int onext = kNumOffsets;  // the offset after o
         if (o < kNumOffsets) {
-            const AT* src = Asw + (size_t)o * NKC * CH;
+            const float2* src = Asw + (size_t)o * NKC * CH;
             for (int e = tid; e < (WHOLE ? NKC * CH : CH); e += NT) abuf[0][e] = src[e];
             has_cur = load_src(o, scur);
             if (has_cur) load_b(scur, 0, bcur);
@@ -621,83 +567,57 @@ __global__ void __launch_bounds__(W * 64) k_m2l_mfma(int np, int ntiles, const i
             // operator prefetch: chunk c of the next offset (WHOLE), else the next item's chunk
             const int pf_o = WHOLE ? onext : on;
             const int pf_c = WHOLE ? c : cn;
-            AT pre[PER];
+            float2 pre[PER];
             if (pf_o < kNumOffsets) {
-                const AT* src = Asw + ((size_t)pf_o * NKC + pf_c) * CH;
+                const float2* src = Asw + ((size_t)pf_o * NKC + pf_c) * CH;
 #pragma unroll
                 for (int i = 0; i < PER; ++i) {
                     const int e = tid + NT * i;
-                    pre[i] = (e < CH) ? src[e] : AT{};
+                    pre[i] = (e < CH) ? src[e] : float2{0.f, 0.f};
                 }
             }
             // sources and B of the next item
             const bool nxt_has = (cn == 0) ? has_next : has_cur;
-            if (on < kNumOffsets && nxt_has) {
-                if (cn == 0) load_b(snext, 0, bnext);
-                else load_b(scur, cn, bnext);
-            }
+            if (on < kNumOffsets && nxt_has) load_b(cn == 0 ? snext : scur, cn, bnext);
             if (has_cur) {
-                const AT* ab = abuf[buf] + (WHOLE ? c * CH : 0) + lane;
-                if constexpr (MIX) {
-                    float bh[CB][KC], bl[CB][KC];
+                const float2* ab = abuf[buf] + (WHOLE ? c * CH : 0) + lane;
+                float bh[KC], bl[KC];
 #pragma unroll
-                    for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-                        for (int kk = 0; kk < KC; ++kk) {
-                            bh[cb][kk] = (float)bcur[cb][kk];
-                            bl[cb][kk] = (float)(bcur[cb][kk] - (double)bh[cb][kk]);
-                        }
-#pragma unroll
-                    for (int kk = 0; kk < KC; ++kk)
-#pragma unroll
-                        for (int rb = 0; rb < RBH; ++rb) {
-                            if (RS > 1 && rb0 + rb >= RB) continue;  // (the last wave's short share)
-                            const float2 a = ab[((rb0 + rb) * KC + kk) * 64];
-#pragma unroll
-                            for (int cb = 0; cb < CB; ++cb) {
-                                acc[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, bh[cb][kk], acc[cb][rb], 0, 0, 0);
-                                acc[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, bl[cb][kk], acc[cb][rb], 0, 0, 0);
-                                acc[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, bh[cb][kk], acc[cb][rb], 0, 0, 0);
-                            }
-                        }
-                } else {
-#pragma unroll
-                    for (int kk = 0; kk < KC; ++kk)
-#pragma unroll
-                        for (int rb = 0; rb < RBH; ++rb) {
-                            if (RS > 1 && rb0 + rb >= RB) continue;
-                            const double a = ab[((rb0 + rb) * KC + kk) * 64];
-#pragma unroll
-                            for (int cb = 0; cb < CB; ++cb)
-                                acc[cb][rb] =
-                                    __builtin_amdgcn_mfma_f64_16x16x4f64(a, bcur[cb][kk], acc[cb][rb], 0, 0, 0);
-                        }
+                for (int kk = 0; kk < KC; ++kk) {
+                    bh[kk] = (float)bcur[kk];
+                    bl[kk] = (float)(bcur[kk] - (double)bh[kk]);
                 }
+#pragma unroll
+                for (int kk = 0; kk < KC; ++kk)
+#pragma unroll
+                    for (int rb = 0; rb < RBH; ++rb) {
+                        if (RS > 1 && rb0 + rb >= RB) continue;  // (the last wave's short share)
+                        const float2 a = ab[((rb0 + rb) * KC + kk) * 64];
+                        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, bh[kk], acc[rb], 0, 0, 0);
+                        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, bl[kk], acc[rb], 0, 0, 0);
+                        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, bh[kk], acc[rb], 0, 0, 0);
+                    }
                 if (TR > 0 && tail) {
-                    const AT* tb = abuf[buf] + (WHOLE ? c * CH : 0) + RB * KC * 64 + kq;
+                    const float2* tb = abuf[buf] + (WHOLE ? c * CH : 0) + RB * KC * 64 + kq;
 #pragma unroll
                     for (int kk = 0; kk < KC; ++kk)
 #pragma unroll
                         for (int tr = 0; tr < TR; ++tr) {
-                            const double a = a_value(tb[(tr * KC + kk) * 4]);
-#pragma unroll
-                            for (int cb = 0; cb < CB; ++cb) tacc[cb][tr] = fma(a, bcur[cb][kk], tacc[cb][tr]);
+                            const float2 a = tb[(tr * KC + kk) * 4];
+                            tacc[tr] = fma((double)a.x + (double)a.y, bcur[kk], tacc[tr]);
                         }
                 }
-                if constexpr (MIX)
-                    if (cn == 0)  // offset o done: fold its FP32 sums into FP64
+                if (cn == 0)  // offset o done: fold its FP32 sums into FP64
 #pragma unroll
-                        for (int cb = 0; cb < CB; ++cb)
+                    for (int rb = 0; rb < RBH; ++rb)
 #pragma unroll
-                            for (int rb = 0; rb < RBH; ++rb)
-#pragma unroll
-                                for (int r = 0; r < 4; ++r) {
-                                    accd[cb][rb][r] += (double)acc[cb][rb][r];
-                                    acc[cb][rb][r] = 0.f;
-                                }
+                        for (int r = 0; r < 4; ++r) {
+                            accd[rb][r] += (double)acc[rb][r];
+                            acc[rb][r] = 0.f;
+                        }
             }
             if (pf_o < kNumOffsets) {
-                AT* dst = abuf[buf ^ 1] + (WHOLE ? pf_c * CH : 0);
+                float2* dst = abuf[buf ^ 1] + (WHOLE ? pf_c * CH : 0);
 #pragma unroll
                 for (int i = 0; i < PER; ++i) {
                     const int e = tid + NT * i;
@@ -709,16 +629,13 @@ __global__ void __launch_bounds__(W * 64) k_m2l_mfma(int np, int ntiles, const i
                 buf ^= 1;
             }
             if (cn == 0 && on < kNumOffsets) {
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb) scur[cb] = snext[cb];
+                scur = snext;
                 has_cur = has_next;
                 onext = next_present(on);
                 has_next = load_src(onext, snext);
             }
 #pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-                for (int kk = 0; kk < KC; ++kk) bcur[cb][kk] = bnext[cb][kk];
+            for (int kk = 0; kk < KC; ++kk) bcur[kk] = bnext[kk];
             o = on;
             c = cn;
         }
@@ -726,34 +643,24 @@ __global__ void __launch_bounds__(W * 64) k_m2l_mfma(int np, int ntiles, const i
     if constexpr (TR > 0) {
         // (kq 0 + kq 1) + (kq 2 + kq 3), in every lane
 #pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-            for (int tr = 0; tr < TR; ++tr) {
-                tacc[cb][tr] += __shfl_xor(tacc[cb][tr], 16, 64);
-                tacc[cb][tr] += __shfl_xor(tacc[cb][tr], 32, 64);
-            }
+        for (int tr = 0; tr < TR; ++tr) {
+            tacc[tr] += __shfl_xor(tacc[tr], 16, 64);
+            tacc[tr] += __shfl_xor(tacc[tr], 32, 64);
+        }
     }
+    if (!valid) return;
+    double* __restrict__ out = L + (size_t)order[rank] * S;
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-        if (!valid[cb]) continue;
-        const int t = order[rank[cb]];
+    for (int rb = 0; rb < RBH; ++rb)
 #pragma unroll
-        for (int rb = 0; rb < RBH; ++rb)
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * (rb0 + rb) + 4 * kq + r;
+            if (rb0 + rb < RB && row < S) out[row] = accd[rb][r];
+        }
+    if constexpr (TR > 0)
+        if (tail && kq == 0)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                // D(i, j) of lane j + 16 kq, register r: i = kq + 4r (f64), 4kq + r (f32)
-                const int R0 = 16 * (rb0 + rb);
-                const int row = MIX ? R0 + 4 * kq + r : R0 + kq + 4 * r;
-                if (rb0 + rb < RB && row < S) {
-                    if constexpr (MIX) L[(size_t)t * S + row] = accd[cb][rb][r];
-                    else L[(size_t)t * S + row] = acc[cb][rb][r];
-                }
-            }
-        if constexpr (TR > 0)
-            if (tail && kq == 0)
-#pragma unroll
-                for (int tr = 0; tr < TR; ++tr) L[(size_t)t * S + 16 * RB + tr] = tacc[cb][tr];
-    }
+            for (int tr = 0; tr < TR; ++tr) out[16 * RB + tr] = tacc[tr];
 }
 
 // ---- M2L on bf16 matrix cores with three-piece split operands -------------------
@@ -962,7 +869,8 @@ __global__ void __launch_bounds__(W * 64) k_m2l_bf16(int np, int ntiles, const i
 // per 16 parents and 16-row block b; wave c makes block b of the rows of class c.
 //   M2M (FmmExpansions3D.hpp:242-265): the children's multipoles are
 //     transformed over the octants into W (LDS), row class c takes
-//     W_{c ^ class(k)}[k]; overwrites Mhat[parent].
+//     W_{c ^ class(k)}[k]; overwrites Mhat[parent] (and its packed copy Mp for
+//     the FP64 M2L, when non-null).
 //   L2L (:307-330): the products of the parent's local are kept apart by
 //     column class, and their transform over the classes gives all children's
 //     rows; adds into Lhat[child].
@@ -1013,8 +921,9 @@ template <int P>
 __global__ void __launch_bounds__(kLevelWaves * 64) k_m2m(int n, const int* __restrict__ tgt,
                                                          const int* __restrict__ child_first,
                                                          const unsigned char* __restrict__ mask,
-                                                         const double* __restrict__ A, double* __restrict__ M) {
-    constexpr int S = nterms(P);
+                                                         const double* __restrict__ A, double* __restrict__ M,
+                                                         double* __restrict__ Mp) {
+    constexpr int S = nterms(P), SP = m2l_pack(P);
     constexpr SymTab T = make_sym_tab(P);
     constexpr int NQ = T.nq, RB = T.rb, G = m2m_group_classes(T), ROWS = m2m_group_rows(T, G);
     constexpr int NT = kLevelWaves * 64, PER = (16 * ROWS + NT - 1) / NT;
@@ -1078,10 +987,15 @@ __global__ void __launch_bounds__(kLevelWaves * 64) k_m2m(int n, const int* __re
     }
     const int t = box[j];
     if (t < 0) return;
+    if (Mp && b == 0)
+        for (int e = 4 * c + kq; e < kPack<P>.npad; e += 4 * kLevelWaves) Mp[(size_t)t * SP + kPack<P>.pads[e]] = 0.0;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int e = 16 * b + kq + 4 * r;
-        if (e < T.cnt[c]) M[(size_t)t * S + kSymTab<P>.krow[4 * kSymTab<P>.kfirst[c] + e]] = acc[r];
+        if (e >= T.cnt[c]) continue;
+        const int row = kSymTab<P>.krow[4 * kSymTab<P>.kfirst[c] + e];
+        M[(size_t)t * S + row] = acc[r];
+        if (Mp) Mp[(size_t)t * SP + kPack<P>.kpos[row]] = acc[r];
     }
 }
 
@@ -1545,45 +1459,62 @@ const int* p2p_order(Pool& pool, hipStream_t s, const TreeView& t, bool reserve_
     return sb.val[radix_sort(sb, nl, 0, 1, s)];
 }
 
-// M2L preparation: the transposed source table srcT[row * np + rank] (rank:
-// the target's position in the M2L order, row: src_row of the offset for the
-// target's parities; -1 where it has no source at that offset) and the
-// per-tile offset presence table.
-void m2l_prep(hipStream_t s, const TreeView& t, int np, int ntiles, const int* tstart, int* srcT, int* present) {
-    const int nb = t.nb;
-    hipLaunchKernelGGL(k_zero_int, dim3(blocks((long long)ntiles * kNumOffsets)), dim3(kT), 0, s, present,
-                       (size_t)ntiles * kNumOffsets);
-    hipLaunchKernelGGL(k_m2l_src, dim3(xcd_grid((nb + kSrcTargets - 1) / kSrcTargets)), dim3(kT), 0, s, nb, np,
-                       t.m2l_order,
-                       t.vl, t.nv, t.ic, srcT, tstart, ntiles, present);
+// The packed multipoles of the FP64 M2L (row nb stays zero).
+template <int P>
+double* packed_multipoles(Pool& pool, const TreeView& t) {
+    constexpr int SP = m2l_pack(P);
+    return pool.get<double>("Mpack", ((size_t)t.nb + 1) * SP);
 }
 
-// The M2L buffers of order P and precision prec, taken from the pool under
-// the names run<P> uses.
+// The M2L buffers of order P and precision prec, taken from the pool.
 template <int P>
-void m2l_prep_for(Pool& pool, hipStream_t s, const TreeView& t, int prec, const Shapes& sh) {
-    const int nb = t.nb, np = nb;
-    (void)prec;
-    const int TILE = m2l_tile_targets(P, prec, sh.m2l_waves);
-    if (TILE != 256 && TILE != 128) throw std::runtime_error("M2L tile size without a plan");
-    const int* tstart = TILE == 256 ? t.m2l_tiles256 : t.m2l_tiles128;
-    const int ntiles = TILE == 256 ? t.m2l_ntiles256 : t.m2l_ntiles128;
-    int* srcT = pool.get<int>("m2l_srcT", (size_t)kSrcRows * np);
-    int* present = pool.get<int>("m2l_present", (size_t)ntiles * kNumOffsets);
-    m2l_prep(s, t, np, ntiles, tstart, srcT, present);
+struct M2LBufs {
+    static constexpr int kPackN = m2l_pack(P);
+    int np, ntiles;
+    const int* tstart;
+    int *srcT, *present;
+    double* Mp;  // packed multipoles (FP64 form), row nb all zeros
+    M2LBufs(Pool& pool, const TreeView& t, int prec) {
+        const bool fp64 = m2l_form(prec) == kPrecFP64;
+        np = t.nb;
+        tstart = t.m2l_tiles;
+        ntiles = t.m2l_ntiles;
+        srcT = pool.get<int>("m2l_srcT", (size_t)(kSrcRows + 1) * np);
+        present = pool.get<int>("m2l_present", (size_t)ntiles * (fp64 ? src_slots<m2l_axes(P)>() : kNumOffsets));
+        Mp = fp64 ? packed_multipoles<P>(pool, t) : nullptr;
+    }
+};
+
+// M2L preparation: the transposed source table srcT[row * np + rank] (rank:
+// the target's position in the M2L order, row: src_row of the offset for the
+// target's parities; -1 where it has no source at that offset), the per-tile
+// slot presence table and the zero multipole of the FP64 form.
+template <int P>
+void m2l_prep(Pool& pool, hipStream_t s, const TreeView& t, int prec) {
+    const M2LBufs<P> m(pool, t, prec);
+    const dim3 g(xcd_grid((t.nb + kSrcTargets - 1) / kSrcTargets)), b(kT);
+    auto go = [&](auto nx) {
+        constexpr int NX = decltype(nx)::value;
+        const size_t n = (size_t)m.ntiles * src_slots<NX>();
+        hipLaunchKernelGGL(k_zero_int, dim3(blocks((long long)n)), dim3(kT), 0, s, m.present, n);
+        hipLaunchKernelGGL(k_m2l_src<NX>, g, b, 0, s, t.nb, m.np, t.m2l_order, t.vl, t.nv, t.ic, m.srcT, m.tstart,
+                           m.ntiles, m.present, m.Mp ? m.Mp + (size_t)t.nb * m.kPackN : nullptr, (int)m.kPackN);
+    };
+    if (m.Mp) go(std::integral_constant<int, m2l_axes(P)>{});
+    else go(std::integral_constant<int, -1>{});
 }
 
 // P2M into M, then M2M level by level (upward pass).
 template <int P>
-void upward(hipStream_t s, const TreeView& t, const TreeMeta& meta, const FmmTables& tab, double* M, hipEvent_t e0,
-            hipEvent_t e1) {
+void upward(hipStream_t s, const TreeView& t, const TreeMeta& meta, const FmmTables& tab, double* M, double* Mp,
+            hipEvent_t e0, hipEvent_t e1) {
     if (e0) AFMM_CHECK(hipEventRecord(e0, s));
-    hipLaunchKernelGGL((k_accumulate<P, 0>), dim3(xcd_chunk_grid(t.nleaves)), dim3(64), 0, s, t, M);
+    hipLaunchKernelGGL((k_accumulate<P, 0>), dim3(xcd_chunk_grid(t.nleaves)), dim3(64), 0, s, t, M, Mp);
     for (int l = t.max_level - 1; l >= 0; --l) {
         const int off = meta.nonleaf_off[l], cnt = meta.nonleaf_off[l + 1] - off;
         if (cnt > 0)
             hipLaunchKernelGGL(k_m2m<P>, dim3((cnt + 15) / 16, make_sym_tab(P).rb), dim3(kLevelWaves * 64), 0, s, cnt,
-                               t.nonleaf_ids + off, t.child_first, t.child_mask, tab.m2m_sw, M);
+                               t.nonleaf_ids + off, t.child_first, t.child_mask, tab.m2m_sw, M, Mp);
     }
     if (e1) AFMM_CHECK(hipEventRecord(e1, s));
 }
@@ -1594,50 +1525,33 @@ void upward(hipStream_t s, const TreeView& t, const TreeMeta& meta, const FmmTab
 template <int P>
 void m2l_launch(Pool& pool, hipStream_t s, const TreeView& t, const FmmTables& tab, int prec, const Shapes& sh,
                 hipEvent_t e0, hipEvent_t e1) {
-    constexpr int S = nterms(P);
+    constexpr int S = nterms(P), KB = m2l_bf_kb(S);
     const int form = m2l_form(prec);
-    const int nb = t.nb, np = nb;
+    const int nb = t.nb;
     double* M = pool.get<double>("Mexp", (size_t)nb * S);
     double* L = pool.get<double>("Lexp", (size_t)nb * S);
-    const int TILE = m2l_tile_targets(P, prec, sh.m2l_waves);
-    if (TILE != 256 && TILE != 128) throw std::runtime_error("M2L tile size without a plan");
-    const int* tstart = TILE == 256 ? t.m2l_tiles256 : t.m2l_tiles128;
-    const int ntiles = TILE == 256 ? t.m2l_ntiles256 : t.m2l_ntiles128;
-    const int* srcT = pool.get<int>("m2l_srcT", (size_t)kSrcRows * np);
-    const int* present = pool.get<int>("m2l_present", (size_t)ntiles * kNumOffsets);
-    uint4* Mbf = form == kPrecMixedBf16 ? pool.get<uint4>("m2l_Mbf", (size_t)nb * m2l_bf_kb(S) * kBfPieces * 4)
-                                        : nullptr;
-    if (form == kPrecMixedBf16) {
-        constexpr int KB = m2l_bf_kb(S);
+    const M2LBufs<P> m(pool, t, prec);
+    uint4* Mbf = form == kPrecMixedBf16 ? pool.get<uint4>("m2l_Mbf", (size_t)nb * KB * kBfPieces * 4) : nullptr;
+    if (form == kPrecMixedBf16)
         hipLaunchKernelGGL(k_split_bf16<P>, dim3(blocks((long long)nb * KB * 4)), dim3(kT), 0, s, nb, M, Mbf);
-    }
     if (e0) AFMM_CHECK(hipEventRecord(e0, s));
-    auto launch_m2l = [&](auto wtag) {
-        constexpr int W = decltype(wtag)::value;
-        const dim3 g(xcd_grid(ntiles)), b(W * 64);
-        if (form == kPrecMixedBf16)
-            hipLaunchKernelGGL((k_m2l_bf16<P, W>), g, b, 0, s, np, ntiles, tstart, t.m2l_order, t.ic, srcT, present,
-                               tab.m2l_bf, Mbf, L);
-        else if (form == kPrecMixed)
-            hipLaunchKernelGGL((k_m2l_mfma<P, true, W>), g, b, 0, s, np, ntiles, tstart, t.m2l_order, t.ic, srcT,
-                               present, tab.m2l_hl, M, L);
-        else if constexpr (W == 16 && m2l_row_split(P, false, W) == 1) {
-            // tiles of 16 or 32 targets (small trees): four or two waves per block
-            if (t.m2l_t256 <= 16)
-                hipLaunchKernelGGL((k_m2l_mfma<P, false, W, 4>), g, b, 0, s, np, ntiles, tstart, t.m2l_order, t.ic, srcT,
-                                   present, tab.m2l_sw, M, L);
-            else if (t.m2l_t256 <= 32)
-                hipLaunchKernelGGL((k_m2l_mfma<P, false, W, 2>), g, b, 0, s, np, ntiles, tstart, t.m2l_order, t.ic, srcT,
-                                   present, tab.m2l_sw, M, L);
+    if (form == kPrecFP64) {
+        m2l_fp64(s, P, M2LArgs{m.np, m.ntiles, t.m2l_tile, m.tstart, t.m2l_order, t.ic, m.srcT, m.present, tab.m2l_sw,
+                               m.Mp, L});
+    } else {
+        auto go = [&](auto wtag) {
+            constexpr int W = decltype(wtag)::value;
+            const dim3 g(xcd_grid(m.ntiles)), b(W * 64);
+            if (form == kPrecMixedBf16)
+                hipLaunchKernelGGL((k_m2l_bf16<P, W>), g, b, 0, s, m.np, m.ntiles, m.tstart, t.m2l_order, t.ic, m.srcT,
+                                   m.present, tab.m2l_bf, Mbf, L);
             else
-                hipLaunchKernelGGL((k_m2l_mfma<P, false, W>), g, b, 0, s, np, ntiles, tstart, t.m2l_order, t.ic, srcT,
-                                   present, tab.m2l_sw, M, L);
-        } else
-            hipLaunchKernelGGL((k_m2l_mfma<P, false, W>), g, b, 0, s, np, ntiles, tstart, t.m2l_order, t.ic, srcT,
-                               present, tab.m2l_sw, M, L);
-    };
-    if (sh.m2l_waves == 16) launch_m2l(std::integral_constant<int, 16>{});
-    else launch_m2l(std::integral_constant<int, 8>{});
+                hipLaunchKernelGGL((k_m2l_split<P, W>), g, b, 0, s, m.np, m.ntiles, m.tstart, t.m2l_order, t.ic,
+                                   m.srcT, m.present, tab.m2l_hl, M, L);
+        };
+        if (sh.m2l_waves == 16) go(std::integral_constant<int, 16>{});
+        else go(std::integral_constant<int, 8>{});
+    }
     if (e1) AFMM_CHECK(hipEventRecord(e1, s));
 }
 
@@ -1647,7 +1561,7 @@ void m2l_launch(Pool& pool, hipStream_t s, const TreeView& t, const FmmTables& t
 template <int P>
 void far_passes(Pool& pool, hipStream_t s, const TreeView& t, const double* M, double* Lx, double* farw,
                 double* fpotw, hipEvent_t x_done = nullptr, hipEvent_t w_done = nullptr) {
-    if (Lx) hipLaunchKernelGGL((k_accumulate<P, 2>), dim3(xcd_chunk_grid(t.nb)), dim3(64), 0, s, t, Lx);
+    if (Lx) hipLaunchKernelGGL((k_accumulate<P, 2>), dim3(xcd_chunk_grid(t.nb)), dim3(64), 0, s, t, Lx, nullptr);
     if (x_done) AFMM_CHECK(hipEventRecord(x_done, s));
     if (farw) {
         const int* ord = m2p_order(pool, s, t, m2p_groups<P>(), false);
@@ -1672,14 +1586,7 @@ void run(Pool& pool, hipStream_t s, const TreeView& t, const TreeMeta& meta, con
     double* L = pool.get<double>("Lexp", (size_t)nb * S);
     double* far = pool.get<double>("far", 3 * (size_t)t.n);
     double* fpot = phi ? pool.get<double>("farpot", t.n) : nullptr;
-    // M2L targets in (octant, level) order, tiles cut inside octant groups
-    const int TILE = m2l_tile_targets(P, prec, sh.m2l_waves);
-    if (TILE != 256 && TILE != 128) throw std::runtime_error("M2L tile size without a plan");
-    const int* tstart = TILE == 256 ? t.m2l_tiles256 : t.m2l_tiles128;
-    const int ntiles = TILE == 256 ? t.m2l_ntiles256 : t.m2l_ntiles128;
-    const int np = nb;
-    int* srcT = pool.get<int>("m2l_srcT", (size_t)kSrcRows * np);
-    int* present = pool.get<int>("m2l_present", (size_t)ntiles * kNumOffsets);
+    const M2LBufs<P> m2l(pool, t, prec);
     uint4* Mbf = form == kPrecMixedBf16 ? pool.get<uint4>("m2l_Mbf", (size_t)nb * m2l_bf_kb(S) * kBfPieces * 4)
                                         : nullptr;
     (void)Mbf;  // (sized here for the capture; m2l_launch takes it)
@@ -1710,9 +1617,9 @@ void run(Pool& pool, hipStream_t s, const TreeView& t, const TreeMeta& meta, con
     };
     const bool p2p_after_m2l = form == kPrecMixedBf16;
     if (split && !p2p_after_m2l && !side.p2p_launched) fork_p2p();
-    if (!side.upward_launched) upward<P>(s, t, meta, tab, M, ev ? ev[0] : nullptr, ev ? ev[1] : nullptr);
+    if (!side.upward_launched) upward<P>(s, t, meta, tab, M, m2l.Mp, ev ? ev[0] : nullptr, ev ? ev[1] : nullptr);
     if (!side.m2l_launched) {
-        if (!side.prep_done) m2l_prep(s, t, np, ntiles, tstart, srcT, present);
+        if (!side.prep_done) m2l_prep<P>(pool, s, t, prec);
         if (side.upward_launched && side.up_done) AFMM_CHECK(hipStreamWaitEvent(s, side.up_done, 0));  // M done
         m2l_launch<P>(pool, s, t, tab, prec, sh, ev ? ev[5] : nullptr, nullptr);
     }
@@ -1725,7 +1632,7 @@ void run(Pool& pool, hipStream_t s, const TreeView& t, const TreeMeta& meta, con
         AFMM_CHECK(hipStreamWaitEvent(s, side.x_done, 0));
         if (Lx) hipLaunchKernelGGL(k_add_x, dim3(blocks((long long)nb * S)), dim3(kT), 0, s, nb, S, t.x_off, Lx, L);
     } else if (t.n_x > 0) {
-        hipLaunchKernelGGL((k_accumulate<P, 1>), dim3(xcd_chunk_grid(nb)), dim3(64), 0, s, t, L);
+        hipLaunchKernelGGL((k_accumulate<P, 1>), dim3(xcd_chunk_grid(nb)), dim3(64), 0, s, t, L, nullptr);
     }
     for (int l = 0; l < t.max_level; ++l) {
         const int off = meta.nonleaf_off[l], cnt = meta.nonleaf_off[l + 1] - off;
@@ -1759,12 +1666,15 @@ void run(Pool& pool, hipStream_t s, const TreeView& t, const TreeMeta& meta, con
 
 }  // namespace
 
-void run_upward(Pool& pool, hipStream_t s, const TreeView& tv, const TreeMeta& meta, int p, const FmmTables& tab,
-                hipEvent_t e0, hipEvent_t e1) {
+void run_upward(Pool& pool, hipStream_t s, const TreeView& tv, const TreeMeta& meta, int p, int prec,
+                const FmmTables& tab, hipEvent_t e0, hipEvent_t e1) {
     double* M = pool.get<double>("Mexp", (size_t)tv.nb * nterms(p));
+    const bool fp64 = m2l_form(prec) == kPrecFP64;
     switch (p) {
 #define AFMM_CASE(PP) \
-    case PP: upward<PP>(s, tv, meta, tab, M, e0, e1); return;
+    case PP: \
+        upward<PP>(s, tv, meta, tab, M, fp64 ? packed_multipoles<PP>(pool, tv) : nullptr, e0, e1); \
+        return;
         AFMM_CASE(1) AFMM_CASE(2) AFMM_CASE(3) AFMM_CASE(4) AFMM_CASE(5) AFMM_CASE(6)
         AFMM_CASE(7) AFMM_CASE(8) AFMM_CASE(9) AFMM_CASE(10) AFMM_CASE(11) AFMM_CASE(12)
         AFMM_CASE(13) AFMM_CASE(14) AFMM_CASE(15) AFMM_CASE(16)
@@ -1773,10 +1683,19 @@ void run_upward(Pool& pool, hipStream_t s, const TreeView& tv, const TreeMeta& m
     throw std::runtime_error("unsupported expansion order");
 }
 
-void run_m2l_prep(Pool& pool, hipStream_t s, const TreeView& tv, int p, int prec, const Shapes& sh) {
+M2LTileRule m2l_tile_rule(int p, int prec, int waves) {
+    const int form = m2l_form(prec);
+    if (form == kPrecFP64)
+        return M2LTileRule{m2l_columns(p) == 2 && waves == 16 ? 256 : 128, true, m2l_workgroups(p)};
+    // the mixed forms: 16 targets per wave, or per two of 16 waves (split FP32)
+    const int most = waves / (form == kPrecMixed && waves == 16 ? 2 : 1) * 16;
+    return M2LTileRule{most, most == 256, 1};
+}
+
+void run_m2l_prep(Pool& pool, hipStream_t s, const TreeView& tv, int p, int prec) {
     switch (p) {
 #define AFMM_CASE(PP) \
-    case PP: m2l_prep_for<PP>(pool, s, tv, prec, sh); return;
+    case PP: m2l_prep<PP>(pool, s, tv, prec); return;
         AFMM_CASE(1) AFMM_CASE(2) AFMM_CASE(3) AFMM_CASE(4) AFMM_CASE(5) AFMM_CASE(6)
         AFMM_CASE(7) AFMM_CASE(8) AFMM_CASE(9) AFMM_CASE(10) AFMM_CASE(11) AFMM_CASE(12)
         AFMM_CASE(13) AFMM_CASE(14) AFMM_CASE(15) AFMM_CASE(16)

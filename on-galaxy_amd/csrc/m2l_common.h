@@ -1,0 +1,41 @@
+// ============================================================================
+// m2l_common.h -- device helpers shared by the M2L kernels (fmm.hip,
+// m2l_fp64.hip): XCD-aware workgroup order and the M2L source table's rows.
+// ============================================================================
+#pragma once
+
+#include "afmm_internal.h"
+#include "afmm_math.h"
+
+namespace afmm {
+
+// ---- XCD-aware workgroup order ------------------------------------------------
+// MI355X deals workgroups round-robin to its 8 XCDs, each with its own L2.
+// Kernels whose neighbouring work items (tiles or leaves in tree order) read
+// the same neighbour data launch xcd_grid(n) workgroups and take item
+// xcd_item(): each XCD then runs one contiguous range of items, in order, and
+// the shared reads hit its L2. Items >= n return at once.
+constexpr int kXcds = 8;
+inline int xcd_grid(int n) { return (n + kXcds - 1) / kXcds * kXcds; }
+__device__ __forceinline__ int xcd_item() {
+    return (int)(blockIdx.x % kXcds) * (int)(gridDim.x / kXcds) + (int)(blockIdx.x / kXcds);
+}
+
+// Source-table rows: a target at integer coordinate 2 P + c (c = 0 or 1 per
+// axis, the parities par = 4 cx + 2 cy + cz) meets its V-list sources, the
+// children of its parent's colleagues P - 1 .. P + 1 that are not adjacent,
+// only at offsets d = ic(target) - ic(source) in [c - 3, c + 2]: 6 of the 7
+// values per axis, 216 of the 343 offsets. Row of offset index oi
+// (offset_index) for parities par, or -1 where the target cannot meet it.
+__device__ __forceinline__ int src_row(int oi, int par) {
+    const int ux = oi / 49 - (par >> 2), uy = (oi / 7) % 7 - ((par >> 1) & 1), uz = oi % 7 - (par & 1);
+    return (unsigned)ux < 6u && (unsigned)uy < 6u && (unsigned)uz < 6u ? (ux * 6 + uy) * 6 + uz : -1;
+}
+__device__ __forceinline__ int ic_parity(const int* __restrict__ ic, int b) {
+    return ((ic[3 * (size_t)b] & 1) << 2) | ((ic[3 * (size_t)b + 1] & 1) << 1) | (ic[3 * (size_t)b + 2] & 1);
+}
+
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+
+}  // namespace afmm

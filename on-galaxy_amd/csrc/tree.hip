@@ -734,26 +734,23 @@ __global__ void __launch_bounds__(kOctCountThreads) k_octant_count(int nb, const
 // derives the tile count from the same counts with m2l_tile_count().
 __host__ __device__ inline int m2l_tiles_of(int cnt, int T) { return (cnt + T - 1) / T; }
 
-// Targets per M2L tile for workgroups of up to `tile` targets: the smallest
-// size whose tiles still fit one per CU, else `tile`. A workgroup's time is
-// set by its busiest SIMD's chain of MFMAs per offset times the offsets, so
-// below a CU's worth of full tiles smaller tiles on more CUs finish sooner:
-// multiples of 64 targets (one 16-target column block per SIMD), and for the
-// 16-wave FP64 workgroups (the 256 plan) also 32 and 16 targets, whose blocks
-// the launch splits by rows over two and four waves (shorter chains).
-int m2l_tile_size(const int* per_octant, int tile, int cus) {
+// Targets per M2L tile under a rule: the smallest allowed size whose tiles
+// still fit the CUs at once, else the largest. A workgroup's time is set by its
+// busiest SIMD's chain of matrix steps per operator times the operators, so
+// below a CU's worth of full tiles smaller tiles on more CUs finish sooner.
+int m2l_tile_size(const int* per_octant, M2LTileRule rule, int cus) {
     auto tiles = [&](int t) {
         int k = 0;
         for (int q = 0; q < 8; ++q)
             if (per_octant[q] > 0) k += m2l_tiles_of(per_octant[q], t);
         return k;
     };
-    if (tile == 256)
+    if (rule.small)
         for (int t : {16, 32})
             if (tiles(t) <= cus) return t;
-    for (int t = 64; t < tile; t += 64)
-        if (tiles(t) <= cus) return t;
-    return tile;
+    for (int t = 64; t < rule.most; t += 64)
+        if (tiles(t) <= cus * rule.per_cu) return t;
+    return rule.most;
 }
 
 // Compute units of the current device (cached per device).
@@ -1248,7 +1245,7 @@ int read_int(const int* d, hipStream_t s) {
 void build_forest(Pool& pool, hipStream_t s, const double* d_pos, const double* d_mass, int nsys,
                   const int* h_sys_off, const double* h_eps_floor, int cap, TreeView& tv, TreeMeta& meta,
                   std::vector<RootInfo>& roots, const TreeHook& on_core, const TreeHook& on_vlists,
-                  hipStream_t ls, hipEvent_t ls_ready, int* levels_hint, int* depth_hint) {
+                  hipStream_t ls, hipEvent_t ls_ready, int* levels_hint, int* depth_hint, M2LTileRule tiles) {
     const int n = h_sys_off[nsys];
     // ---- per-system root cubes: chunks of at most kBBoxChunk bodies of one system
     std::vector<int> hb;  // [cbeg | cend | cfirst(nsys+1) | sys_off(nsys+1)] as one upload
@@ -1622,25 +1619,19 @@ void build_forest(Pool& pool, hipStream_t s, const double* d_pos, const double* 
             hipLaunchKernelGGL(k_fill, dim3(1), dim3(kT), 0, s, tv.m2l_order, nb, 0);
         // M2L tiles (tile starts built on the device from the same counts)
         int tot = 0;
-        tv.m2l_ntiles256 = tv.m2l_ntiles128 = 0;
+        tv.m2l_ntiles = 0;
         const int* per_octant = got.data() + nlev;
-        const int cus = device_cus();
-        const int t256 = m2l_tile_size(per_octant, 256, cus), t128 = m2l_tile_size(per_octant, 128, cus);
-        tv.m2l_t256 = t256;
+        const int ts = m2l_tile_size(per_octant, tiles, device_cus());
+        tv.m2l_tile = ts;
         for (int q = 0; q < 8; ++q) {
             const int c = per_octant[q];
             if (c <= 0) continue;
             tot += c;
-            tv.m2l_ntiles256 += m2l_tiles_of(c, t256);
-            tv.m2l_ntiles128 += m2l_tiles_of(c, t128);
+            tv.m2l_ntiles += m2l_tiles_of(c, ts);
         }
         if (tot != nb) throw std::runtime_error("octant counts do not cover the boxes");
-        tv.m2l_tiles256 = pool.get<int>("m2l_tiles256", tv.m2l_ntiles256 + 1);
-        tv.m2l_tiles128 = pool.get<int>("m2l_tiles128", tv.m2l_ntiles128 + 1);
-        hipLaunchKernelGGL(k_m2l_tile_plan, dim3(1), dim3(kT), 0, s, d_oct_cnt, t256, tv.m2l_ntiles256,
-                           tv.m2l_tiles256);
-        hipLaunchKernelGGL(k_m2l_tile_plan, dim3(1), dim3(kT), 0, s, d_oct_cnt, t128, tv.m2l_ntiles128,
-                           tv.m2l_tiles128);
+        tv.m2l_tiles = pool.get<int>("m2l_tiles", tv.m2l_ntiles + 1);
+        hipLaunchKernelGGL(k_m2l_tile_plan, dim3(1), dim3(kT), 0, s, d_oct_cnt, ts, tv.m2l_ntiles, tv.m2l_tiles);
     }
 
     // ---- colleagues, V, M2L source table

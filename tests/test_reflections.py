@@ -76,3 +76,24 @@ def test_forces_against_oracle(kind, p):
     mx, _ = cabi.rel_err(ref, acc)
     print(f"{kind} p={p}: {mx:.2e}", flush=True)
     assert mx <= 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p", [2, 4, 6, 8, 11, 16])
+def test_batch_tiles_equal_alone(p):
+    """A forest whose M2L runs full tiles gives each system the bits it has
+    alone, where its few boxes run tiles of 16 targets over four waves."""
+    rng = np.random.default_rng(p)
+    sizes = [int(n) for n in rng.integers(1500, 4000, 70)]
+    off = np.concatenate([[0], np.cumsum(sizes)])
+    pos = rng.standard_normal((off[-1], 3))
+    m = rng.uniform(0.5, 1.5, off[-1])
+    s = cabi.product().AdaptiveFMM3D(G=1.0, eps=0.01, p=p, threshold=7)
+    acc = s.computeBatch(pos, m, off)
+    boxes = s.stats()["n_boxes"]
+    assert boxes > 256 * 32  # more than fit tiles of 32 targets on the CUs
+    for q in (0, 33, 69):
+        sl = slice(off[q], off[q + 1])
+        assert np.array_equal(acc[sl], s.computeAccelerations(pos[sl], m[sl])), q
+    s.close()
+    print(f"p={p}: {boxes} boxes", flush=True)
