@@ -114,6 +114,35 @@ AFMM_HD void singular_stream(double x, double y, double z, F&& f) {
     }
 }
 
+// ---- factorial-scaled singular harmonics -----------------------------------------
+// T_n^a = sqrt((n-a)! (n+a)!) S_n^a:
+//   T_0^0 = 1/|v|, T_a^a = (2a-1)(ux + i uy) T_{a-1}^{a-1}, u = v / |v|^2,
+//   T_n^a = (2n-1) uz T_{n-1}^a - ((n-1)^2 - a^2) |v|^-2 T_{n-2}^a,
+// and the gradient of sum M_n^m S_n^m (multipole_grad) has plain sums as its
+// factors of T once the multipole is scaled by fact_scale(n, a): with N = M
+// fact_scale, harmonic (n+1, a) enters x and y through N_n^{a-1} and
+// N_n^{a+1}, and z as -N_n^a (twice for a > 0).
+constexpr double const_sqrt(double x) {  // (constant expressions only: Newton's iteration)
+    double y = x > 1.0 ? x : 1.0;
+    for (int k = 0; k < 80; ++k) y = 0.5 * (y + x / y);
+    return y;
+}
+constexpr double fact_scale(int n, int a) {
+    double f = 1.0;
+    for (int k = 2; k <= n - a; ++k) f *= k;
+    for (int k = 2; k <= n + a; ++k) f *= k;
+    return 1.0 / const_sqrt(f);
+}
+template <int P>
+struct FactScale {
+    double of[nterms(P)];  // by storage index
+    constexpr FactScale() : of{} {
+        for (int n = 0; n <= P; ++n)
+            for (int a = 0; a <= n; ++a)
+                for (int im = 0; im < (a ? 2 : 1); ++im) of[rid(n, a) + im] = fact_scale(n, a);
+    }
+};
+
 // ---- per-point operators ----------------------------------------------------
 // P2M contribution of one body (mass q, scaled offset d from the box centre):
 // Mhat_n^a += q conj(R_n^a(d)).

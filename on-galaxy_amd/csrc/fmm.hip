@@ -236,44 +236,226 @@ __global__ void __launch_bounds__(64) k_accumulate(TreeView t, double* __restric
 }
 
 // ---- M2P over W (AdaptiveFMM3D.hpp:95, FmmExpansions3D.hpp:180-200) --------------
-// One workgroup of kM2PWaves waves per target leaf. Its L = 64 * kM2PWaves lanes
-// form G = L / T lane groups of T = max(n_leaf, L / m2p_groups) lanes (T = L
-// above L bodies); group g handles W entries g, g + G, ... with their
-// multipoles staged in LDS. Partial fields are reduced across groups in a
-// fixed order and added to far[] (and, with POT, the potential to fpot[]).
-// Four waves per leaf rather than one: the W lists are heavy-tailed (a few
-// clustered leaves hold 200-300 entries), and one wave per leaf left those
-// waves running long after the rest of the grid had drained.
-// At p <= 8 the kernel is held to 128 VGPRs (four waves per SIMD; a few bytes
-// spill), measured 5% faster than 143 VGPRs at three waves; above p = 8 that
-// limit spills hundreds of bytes and is not applied.
-constexpr int kM2PWaves = 4;
+// One workgroup per target leaf: its lanes form G groups of T = ceil(n / R)
+// lanes, R bodies per lane; group g handles W entries g, g + G, ... with their
+// multipoles, scaled by fact_scale, staged in LDS (at most GM entries at a
+// time), and the groups' fields are added in a fixed order into far[] (and
+// fpot[]).
+// Bound by FP64 VALU issue and LDS reads: a pair takes the 243 values of the
+// multipole that its three gradient sums touch, and one body per lane asks LDS
+// for them as fast as it delivers. Two bodies share each read and the factors
+// formed from it; a pair then costs 6 FMAs per complex harmonic, 6 operations
+// of its recurrence and 2 of the factors (15 and 6 from the multipole itself).
+// All leaves: 1M, p = 8 680 -> 505 us, 700k, p = 4 221 -> 156, 300k, p = 12
+// 625 -> 407, 120k, p = 16 611 -> 255. Four bodies per lane leave too few waves
+// (652 at 1M with multipole_grad's constants, two 597, one 689); factors
+// precomputed per box (2.4 KB against 0.6 KB staged per entry) took 1037.
+constexpr int kM2PLanes = 256;
+constexpr int m2p_groups(int p) { return p <= 8 ? 32 : 16; }
+// Waves per SIMD that the registers are held to (p = 12: three 407, four 491 us).
+constexpr int m2p_waves(int p) { return p > 8 && p <= 12 ? 3 : 4; }
+__host__ __device__ inline int m2p_per_lane(int n) { return n > 14 ? 2 : 1; }
 template <int P>
-constexpr int m2p_groups() { return P <= 8 ? 32 : 16; }
-template <int P>
-constexpr int m2p_min_waves() { return P <= 8 ? 4 : 1; }
+__constant__ FactScale<P> kFactScale = FactScale<P>();
+
+// Adds the field of one staged multipole m (box scale ih = 1/h) at R offsets d
+// (in units of h) from its centre: multipole_grad of afmm_math.h on the
+// factorial-scaled harmonics.
+template <int P, bool POT, int R>
+__device__ __forceinline__ void m2p_pairs(const double* __restrict__ m, double ih, const double (&d)[R][3],
+                                          double (&f)[R][POT ? 4 : 3]) {
+    double ux[R], uy[R], uz[R], ir2[R], dre[R], dim[R], z0[R], z1[R], p0[R], p1[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const double x = d[r][0], y = d[r][1], z = d[r][2];
+        const double r2 = x * x + y * y + z * z;
+        // 1/|v|: two Newton steps from the 2^-24 hardware estimate
+        double q = __builtin_amdgcn_rsq(r2);
+        q = fma(q * 0.5, fma(-r2 * q, q, 1.0), q);
+        q = fma(q * 0.5, fma(-r2 * q, q, 1.0), q);
+        ir2[r] = q * q;
+        ux[r] = x * ir2[r], uy[r] = y * ir2[r], uz[r] = z * ir2[r];
+        dre[r] = q * (ih * ih);  // (the gradient's box scale; the potential takes it off again)
+        dim[r] = 0.0;
+        z0[r] = z1[r] = p0[r] = p1[r] = 0.0;
+    }
+    // (the offset is opaque from one order to the next, so that the values three
+    // orders share are read again instead of held in registers that spill)
+    int off = 0;
+    // harmonic (n2, a): its factors in the three sums, then the R bodies
+    auto apply = [&](auto nc, auto ac, const double (&re)[R], const double (&im)[R]) {
+        constexpr int n2 = decltype(nc)::value, a = decltype(ac)::value, n = n2 - 1;
+        constexpr bool below = n >= 0 && a >= 1, above = n >= 0 && a + 1 <= n;
+        double br = 0.0, bi = 0.0, ar = 0.0, ai = 0.0;  // N of orders a - 1 and a + 1
+        if constexpr (below) br = m[off + rid(n, a - 1)];
+        if constexpr (below && a > 1) bi = m[off + rid(n, a - 1) + 1];
+        if constexpr (above) ar = m[off + rid(n, a + 1)], ai = m[off + rid(n, a + 1) + 1];
+        // x: (ar - br) re + (bi - ai) im, y: -(ai + bi) re - (ar + br) im
+        const double xr = !below ? ar : above ? ar - br : -br, yi = !below ? ar : above ? ar + br : br;
+        const double yr = below && a > 1 ? (above ? ai + bi : bi) : ai;
+        const double xi = below && a > 1 ? (above ? bi - ai : bi) : -ai;
+        double zr = 0.0, zi = 0.0, vr = 0.0, vi = 0.0;
+        if constexpr (n >= 0 && a <= n) zr = m[off + rid(n, a)];
+        if constexpr (n >= 0 && a <= n && a > 0) zi = m[off + rid(n, a) + 1];
+        if constexpr (POT && n2 <= P) vr = m[off + rid(n2, a)];
+        if constexpr (POT && n2 <= P && a > 0) vi = m[off + rid(n2, a) + 1];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if constexpr (below || above) f[r][0] = fma(xr, re[r], f[r][0]);
+            if constexpr ((below && a > 1) || above) f[r][1] = fma(-yr, re[r], f[r][1]);
+            if constexpr (a > 0 && ((below && a > 1) || above)) f[r][0] = fma(xi, im[r], f[r][0]);
+            if constexpr (a > 0 && (below || above)) f[r][1] = fma(-yi, im[r], f[r][1]);
+            if constexpr (n >= 0 && a <= n) {
+                if constexpr (a == 0) z0[r] = fma(zr, re[r], z0[r]);
+                else z1[r] = fma(-zi, im[r], fma(zr, re[r], z1[r]));
+            }
+            if constexpr (POT && n2 <= P) {
+                if constexpr (a == 0) p0[r] = fma(vr, re[r], p0[r]);
+                else p1[r] = fma(-vi, im[r], fma(vr, re[r], p1[r]));
+            }
+        }
+    };
+    static_for<P + 2>([&](auto ac) {
+        constexpr int a = decltype(ac)::value;
+        asm volatile("" : "+v"(off));
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if constexpr (a == 1) {
+                dim[r] = uy[r] * dre[r];
+                dre[r] = ux[r] * dre[r];
+            } else if constexpr (a > 1) {
+                const double x = (2.0 * a - 1.0) * ux[r], y = (2.0 * a - 1.0) * uy[r];
+                const double re = fma(x, dre[r], -(y * dim[r]));
+                dim[r] = fma(x, dim[r], y * dre[r]);
+                dre[r] = re;
+            }
+        }
+        if constexpr (POT || a > 0) apply(ac, ac, dre, dim);
+        if constexpr (a <= P) {
+            double p2re[R], p2im[R], p1re[R], p1im[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const double z = (2.0 * a + 1.0) * uz[r];
+                p2re[r] = dre[r], p2im[r] = dim[r];
+                p1re[r] = z * dre[r];
+                p1im[r] = a > 0 ? z * dim[r] : 0.0;
+            }
+            apply(std::integral_constant<int, a + 1>{}, ac, p1re, p1im);
+            static_for<P - a>([&](auto kc) {
+                constexpr int n = a + 2 + decltype(kc)::value;
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const double z = (2.0 * n - 1.0) * uz[r], s = double((n - 1) * (n - 1) - a * a) * ir2[r];
+                    const double re = fma(z, p1re[r], -(s * p2re[r]));
+                    p2re[r] = p1re[r], p1re[r] = re;
+                    if constexpr (a > 0) {
+                        const double im = fma(z, p1im[r], -(s * p2im[r]));
+                        p2im[r] = p1im[r], p1im[r] = im;
+                    }
+                }
+                apply(std::integral_constant<int, n>{}, ac, p1re, p1im);
+                if constexpr (P <= 8) __builtin_amdgcn_sched_barrier(0);  // (LDS reads stay near: registers)
+            });
+        }
+    });
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        f[r][2] -= fma(2.0, z1[r], z0[r]);
+        if constexpr (POT) f[r][3] += fma(2.0, p1[r], p0[r]) / ih;
+    }
+}
+
+template <int P, bool POT>
+struct M2PLds {
+    double m[m2p_groups(P)][nterms(P)];
+    double red[POT ? 4 : 3][kM2PLanes];
+};
+
+template <int P, bool POT, bool ADD, int R>
+__device__ __forceinline__ void m2p_leaf(const TreeView& t, int f0, int nt, int wa, int nw,
+                                         const double* __restrict__ M, double* __restrict__ far,
+                                         double* __restrict__ fpot, M2PLds<P, POT>& lds) {
+    constexpr int S = nterms(P), L = kM2PLanes, K = POT ? 4 : 3;
+    const int tid = threadIdx.x;
+    const int T = min(L, (nt + R - 1) / R), G = min(L / T, m2p_groups(P));
+    const int g = tid / T, tl = tid % T;
+    for (int tb = 0; tb < nt; tb += T * R) {
+        double x[R][3], f[R][K];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int i = f0 + min(tb + r * T + tl, nt - 1);  // (lanes past the end repeat the last body)
+            x[r][0] = t.x[i], x[r][1] = t.y[i], x[r][2] = t.z[i];
+#pragma unroll
+            for (int o = 0; o < K; ++o) f[r][o] = 0.0;
+        }
+        for (int e0 = 0; e0 < nw; e0 += G) {
+            const int nq = min(G, nw - e0);
+            __syncthreads();
+            for (int e = tid; e < nq * S; e += L) {
+                const int q = e / S, c = e - q * S;
+                lds.m[q][c] = M[(size_t)t.w_idx[wa + e0 + q] * S + c] * kFactScale<P>.of[c];
+            }
+            __syncthreads();
+            if (g < nq) {
+                const int w = t.w_idx[wa + e0 + g];
+                const double* c = t.cdd + 6 * (size_t)w;
+                const double ih = t.invh[w];
+                double d[R][3];
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        d[r][k] = offset_from(x[r][k], Centre{c[2 * k], c[2 * k + 1]}) * ih;
+                m2p_pairs<P, POT, R>(lds.m[g], ih, d, f);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (G > 1) {
+                __syncthreads();
+#pragma unroll
+                for (int o = 0; o < K; ++o) lds.red[o][tid] = f[r][o];
+                __syncthreads();
+                if (g == 0)
+                    for (int q = 1; q < G; ++q)
+#pragma unroll
+                        for (int o = 0; o < K; ++o) f[r][o] += lds.red[o][q * T + tl];
+            }
+            const int k = tb + r * T + tl;
+            if (g == 0 && k < nt) {
+                const size_t i = (size_t)(f0 + k);
+#pragma unroll
+                for (int o = 0; o < 3; ++o) {
+                    if constexpr (ADD) far[3 * i + o] += f[r][o];
+                    else far[3 * i + o] = f[r][o];
+                }
+                if constexpr (POT) {
+                    if constexpr (ADD) fpot[i] += f[r][3];
+                    else fpot[i] = f[r][3];
+                }
+            }
+        }
+    }
+}
 
 // ADD: far += the field (after L2P wrote far); otherwise far = the field, zero
 // for leaves without W (the separate array L2P adds later; the same sums).
 // order: the leaves by descending work (m2p_order); workgroup k takes leaf
 // order[k], which changes when a leaf runs, not what it sums.
 template <int P, bool POT, bool ADD>
-__global__ void __launch_bounds__(kM2PWaves * 64, m2p_min_waves<P>()) k_m2p(TreeView t, const double* __restrict__ M,
+__global__ void __launch_bounds__(kM2PLanes, m2p_waves(P)) k_m2p(TreeView t, const double* __restrict__ M,
                                                        double* __restrict__ far, double* __restrict__ fpot,
                                                        const int* __restrict__ order) {
-    constexpr int S = nterms(P), L = kM2PWaves * 64, GM = m2p_groups<P>();
-    __shared__ double mw[GM][S];
-    __shared__ double red[4][L];
+    __shared__ __align__(16) M2PLds<P, POT> lds;
     const int item = xcd_chunk_item();
     if (item >= t.nleaves) return;
     const int li = order[item];
     const int wa = t.w_off[li], nw = t.w_off[li + 1] - wa;
     const int b = t.leaf_ids[li];
     const int f = t.seg_first[b], nt = t.seg_count[b];
-    const int tid = threadIdx.x;
     if (nw == 0) {  // no W: a zero field, so that L2P can add farw everywhere
         if constexpr (ADD) return;
-        for (int k = tid; k < nt; k += kM2PWaves * 64) {
+        for (int k = threadIdx.x; k < nt; k += kM2PLanes) {
             const size_t i = (size_t)(f + k);
             far[3 * i] = 0.0;
             far[3 * i + 1] = 0.0;
@@ -282,83 +464,10 @@ __global__ void __launch_bounds__(kM2PWaves * 64, m2p_min_waves<P>()) k_m2p(Tree
         }
         return;
     }
-    const int T = nt > L ? L : max(nt, L / GM);
-    const int Gs = L / T;  // <= GM
-    const int g = tid / T, tl = tid % T;
-    for (int tb = 0; tb < nt; tb += T) {
-        const int i = f + tb + tl;
-        const bool act = g < Gs && tb + tl < nt;
-        const double xi = act ? t.x[i] : 0.0, yi = act ? t.y[i] : 0.0, zi = act ? t.z[i] : 0.0;
-        double fx = 0.0, fy = 0.0, fz = 0.0, fp = 0.0;
-        for (int r = 0; r < nw; r += Gs) {
-            __syncthreads();
-            const int nq = min(Gs, nw - r);
-            for (int e = tid; e < nq * S; e += L) {
-                const int q = e / S, c = e - q * S;
-                mw[q][c] = M[(size_t)t.w_idx[wa + r + q] * S + c];
-            }
-            __syncthreads();
-            if (act && g < nq) {
-                const int w = t.w_idx[wa + r + g];
-                const double* c = t.cdd + 6 * (size_t)w;
-                const double ih = t.invh[w];
-                const double dx = offset_from(xi, Centre{c[0], c[1]}) * ih;
-                const double dy = offset_from(yi, Centre{c[2], c[3]}) * ih;
-                const double dz = offset_from(zi, Centre{c[4], c[5]}) * ih;
-                double gx, gy, gz, pt = 0.0;
-                const double* mg = mw[g];
-                multipole_grad<P, POT>([&](int k) { return mg[k]; }, dx, dy, dz, gx, gy, gz, &pt);
-                const double s2 = ih * ih;
-                fx += gx * s2;
-                fy += gy * s2;
-                fz += gz * s2;
-                if constexpr (POT) fp += pt * ih;
-            }
-        }
-        if (Gs > 1) {
-            __syncthreads();
-            red[0][tid] = fx;
-            red[1][tid] = fy;
-            red[2][tid] = fz;
-            red[3][tid] = fp;
-            __syncthreads();
-            if (g == 0)
-                for (int q = 1; q < Gs; ++q) {
-                    fx += red[0][q * T + tl];
-                    fy += red[1][q * T + tl];
-                    fz += red[2][q * T + tl];
-                    fp += red[3][q * T + tl];
-                }
-        }
-        if (act && g == 0) {
-            if constexpr (ADD) {
-                far[3 * (size_t)i] += fx;
-                far[3 * (size_t)i + 1] += fy;
-                far[3 * (size_t)i + 2] += fz;
-                if constexpr (POT) fpot[i] += fp;
-            } else {
-                far[3 * (size_t)i] = fx;
-                far[3 * (size_t)i + 1] = fy;
-                far[3 * (size_t)i + 2] = fz;
-                if constexpr (POT) fpot[i] = fp;
-            }
-        }
-    }
+    if (m2p_per_lane(nt) == 2) m2p_leaf<P, POT, ADD, 2>(t, f, nt, wa, nw, M, far, fpot, lds);
+    else m2p_leaf<P, POT, ADD, 1>(t, f, nt, wa, nw, M, far, fpot, lds);
 }
 
-// ---- M2L on FP64 matrix cores ------------------------------------------------
-// L_t = sum_{c in V(t)} T[offset(t,c)] M_c with level-independent S x S
-// operators. One wave owns 16 targets (the 16 columns of
-// v_mfma_f64_16x16x4_f64) and loops over the 316 separated offsets; for each
-// offset present in its tile it streams the pre-swizzled operator (A, one
-// contiguous 512-byte fragment per MFMA) against the 16 gathered source
-// multipoles (B, zero where a target has no source at that offset), keeping
-// the 16 x S output tile in accumulators for the whole loop. Targets are
-// ordered by (level, octant) so that a tile shares most of its offset pattern.
-// Operand layouts (CDNA 16x16x4 f64): A[i][k] in lane i + 16k, B[k][j] in lane
-// j + 16k, D[i][j] in lane j + 16(i%4), register i/4 (rows interleave by 4,
-// unlike the f32 16x16x4 form; see ck's mfma_type for f64 16x16x4:
-// group_size 1, num_groups_per_blk 4).
 __global__ void __launch_bounds__(kT) k_zero_int(int* a, size_t n) {
     const size_t i = blockIdx.x * (size_t)kT + threadIdx.x;
     if (i < n) a[i] = 0;
@@ -1404,31 +1513,27 @@ void launch_p2p(hipStream_t s, const TreeView& t, bool mixed, const double* far,
                            order);
 }
 
-// M2P's leaf order: a workgroup's work is its rounds, ceil(n / T) * ceil(w / G)
-// for a leaf of n bodies and w W entries with k_m2p's lane groups (T lanes,
-// G = L / T groups), and the leaves are sorted by descending rounds (capped at
-// 511), stable, so leaves of equal work keep tree order. On the 1M merger the
-// rounds run up to 73 against a mean of 5.2 over the leaves with W, and the
-// heaviest leaves, clustered in tree order, otherwise start late and finish
-// last on their XCD (in a greedy model of the dispatch: a makespan of 108
-// rounds in tree order, 76 heavy first, 70 ideal).
+// M2P's leaf order: a workgroup's work is its rounds of R pairs per lane,
+// ceil(n / (T R)) * ceil(w / G) * R for a leaf of n bodies and w W entries (m2p_leaf),
+// and the leaves are sorted by descending work (capped at 511), stable, so
+// leaves of equal work keep tree order: the heaviest leaves, clustered in tree
+// order, otherwise start late and finish last on their XCD.
 __global__ void __launch_bounds__(kT) k_m2p_work(TreeView t, int groups, uint64_t* __restrict__ khi,
                                                  uint32_t* __restrict__ klo, int* __restrict__ val) {
     const int li = blockIdx.x * kT + threadIdx.x;
     if (li >= t.nleaves) return;
-    constexpr int L = kM2PWaves * 64;
     const int nw = t.w_off[li + 1] - t.w_off[li], nt = t.seg_count[t.leaf_ids[li]];
     int r = 0;
     if (nw > 0) {
-        const int T = nt > L ? L : max(nt, L / groups), G = L / T;
-        r = min((nt + T - 1) / T * ((nw + G - 1) / G), 511);
+        const int R = m2p_per_lane(nt), T = min(kM2PLanes, (nt + R - 1) / R), G = min(kM2PLanes / T, groups);
+        r = min((nt + T * R - 1) / (T * R) * ((nw + G - 1) / G) * R, 511);
     }
     khi[li] = 0;
     klo[li] = (uint32_t)(511 - r);
     val[li] = li;
 }
 
-const int* m2p_order(Pool& pool, hipStream_t s, const TreeView& t, int groups, bool reserve_only) {
+const int* m2p_order(Pool& pool, hipStream_t s, const TreeView& t, int p, bool reserve_only) {
     const int nl = t.nleaves;
     SortBufs sb;
     for (int k = 0; k < 2; ++k) {
@@ -1439,7 +1544,8 @@ const int* m2p_order(Pool& pool, hipStream_t s, const TreeView& t, int groups, b
     sb.hist = pool.get<int>("mw_hist", 512 * (size_t)sort_blocks(nl));
     sb.scan_tmp = pool.get<int>("mw_scan", scan_tmp_ints(512 * sort_blocks(nl) + nl) + 16);
     if (reserve_only) return nullptr;
-    hipLaunchKernelGGL(k_m2p_work, dim3(blocks(nl)), dim3(kT), 0, s, t, groups, sb.khi[0], sb.klo[0], sb.val[0]);
+    hipLaunchKernelGGL(k_m2p_work, dim3(blocks(nl)), dim3(kT), 0, s, t, m2p_groups(p), sb.khi[0], sb.klo[0],
+                       sb.val[0]);
     return sb.val[radix_sort(sb, nl, 0, 1, s)];
 }
 
@@ -1555,6 +1661,15 @@ void m2l_launch(Pool& pool, hipStream_t s, const TreeView& t, const FmmTables& t
     if (e1) AFMM_CHECK(hipEventRecord(e1, s));
 }
 
+// M2P over W on stream s into far (ADD: added) and, when non-null, fpot.
+template <int P, bool ADD>
+void m2p(Pool& pool, hipStream_t s, const TreeView& t, const double* M, double* far, double* fpot) {
+    const dim3 g(xcd_chunk_grid(t.nleaves)), b(kM2PLanes);
+    const int* ord = m2p_order(pool, s, t, P, false);
+    if (fpot) hipLaunchKernelGGL((k_m2p<P, true, ADD>), g, b, 0, s, t, M, far, fpot, ord);
+    else hipLaunchKernelGGL((k_m2p<P, false, ADD>), g, b, 0, s, t, M, far, fpot, ord);
+}
+
 // P2L over X into Lx (then x_done) and M2P over W into farw (then w_done) on
 // stream s; either buffer is null when its lists are empty. They read only the
 // tree, the lists, the bodies and the multipoles, so they can run beside M2L.
@@ -1563,12 +1678,7 @@ void far_passes(Pool& pool, hipStream_t s, const TreeView& t, const double* M, d
                 double* fpotw, hipEvent_t x_done = nullptr, hipEvent_t w_done = nullptr) {
     if (Lx) hipLaunchKernelGGL((k_accumulate<P, 2>), dim3(xcd_chunk_grid(t.nb)), dim3(64), 0, s, t, Lx, nullptr);
     if (x_done) AFMM_CHECK(hipEventRecord(x_done, s));
-    if (farw) {
-        const int* ord = m2p_order(pool, s, t, m2p_groups<P>(), false);
-        const dim3 mg(xcd_chunk_grid(t.nleaves)), mb(kM2PWaves * 64);
-        if (fpotw) hipLaunchKernelGGL((k_m2p<P, true, false>), mg, mb, 0, s, t, M, farw, fpotw, ord);
-        else hipLaunchKernelGGL((k_m2p<P, false, false>), mg, mb, 0, s, t, M, farw, fpotw, ord);
-    }
+    if (farw) m2p<P, false>(pool, s, t, M, farw, fpotw);
     if (w_done) AFMM_CHECK(hipEventRecord(w_done, s));
 }
 
@@ -1600,7 +1710,7 @@ void run(Pool& pool, hipStream_t s, const TreeView& t, const TreeMeta& meta, con
     double* nr = split ? pool.get<double>("near", 3 * (size_t)t.n) : nullptr;
     double* npot = split && phi ? pool.get<double>("nearpot", t.n) : nullptr;
     if (sh.p2p_schedule) p2p_order(pool, s, t, true);  // its buffers too
-    if (t.n_w > 0) m2p_order(pool, s, t, m2p_groups<P>(), true);
+    if (t.n_w > 0) m2p_order(pool, s, t, P, true);
     if (reserve_only) return;
     // P2P needs only the tree and the U lists: on the second stream it runs
     // beside the far-field passes. It is forked before M2L in FP64 (it shares
@@ -1643,12 +1753,7 @@ void run(Pool& pool, hipStream_t s, const TreeView& t, const TreeMeta& meta, con
     if (ev) AFMM_CHECK(hipEventRecord(ev[3], s));
     if (fb) AFMM_CHECK(hipStreamWaitEvent(s, side.w_done, 0));
     hipLaunchKernelGGL(k_far<P>, dim3(blocks(t.n)), dim3(kT), 0, s, t, L, far, fpot, farw, fpotw);
-    if (!fb && t.n_w > 0) {  // M2P in order: added to far after L2P
-        const int* ord = m2p_order(pool, s, t, m2p_groups<P>(), false);
-        const dim3 mg(xcd_chunk_grid(t.nleaves)), mb(kM2PWaves * 64);
-        if (fpot) hipLaunchKernelGGL((k_m2p<P, true, true>), mg, mb, 0, s, t, M, far, fpot, ord);
-        else hipLaunchKernelGGL((k_m2p<P, false, true>), mg, mb, 0, s, t, M, far, fpot, ord);
-    }
+    if (!fb && t.n_w > 0) m2p<P, true>(pool, s, t, M, far, fpot);  // in order: added to far after L2P
     if (split) {
         AFMM_CHECK(hipStreamWaitEvent(s, side.join, 0));
         const dim3 cg(xcd_chunk_grid(t.nleaves)), cb(64);

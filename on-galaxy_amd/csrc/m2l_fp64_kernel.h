@@ -14,23 +14,11 @@
 #pragma once
 
 #include <stdexcept>
-#include <type_traits>
-#include <utility>
 
 #include "m2l_common.h"
 
 namespace afmm {
 namespace {
-
-template <class F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-// f(integral_constant 0), ..., f(integral_constant N - 1)
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
 
 template <int P>
 __constant__ M2LPlan kPlan = make_m2l_plan(P);
