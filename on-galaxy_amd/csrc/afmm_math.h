@@ -135,13 +135,60 @@ constexpr double fact_scale(int n, int a) {
 }
 template <int P>
 struct FactScale {
-    double of[nterms(P)];  // by storage index
-    constexpr FactScale() : of{} {
+    double of[nterms(P)], inv[nterms(P)];  // by storage index, and the reciprocals
+    constexpr FactScale() : of{}, inv{} {
         for (int n = 0; n <= P; ++n)
             for (int a = 0; a <= n; ++a)
-                for (int im = 0; im < (a ? 2 : 1); ++im) of[rid(n, a) + im] = fact_scale(n, a);
+                for (int im = 0; im < (a ? 2 : 1); ++im) {
+                    of[rid(n, a) + im] = fact_scale(n, a);
+                    inv[rid(n, a) + im] = 1.0 / fact_scale(n, a);
+                }
     }
 };
+
+
+// p2l_point and p2m_point without their coefficients' scale: add(k, v) collects
+// the terms of Lhat / fact_scale (singular: q T conjugated), and of Mhat
+// fact_scale (regular: q U conjugated, U = R fact_scale with U_a^a = (x + iy) /
+// (2a) U_{a-1}^{a-1} and (n^2 - a^2) U_n^a = (2n-1) z U_{n-1}^a - r^2 U_{n-2}^a).
+// qr: q / |d| (singular) or q; u, w: d / |d|^2 and |d|^-2, or d and |d|^2.
+template <int P, bool SINGULAR, class Acc>
+AFMM_HD void point_terms(double qr, double ux, double uy, double uz, double w, Acc&& add) {
+    auto put = [&](int n, int a, double re, double im) {
+        add(rid(n, a), re);
+        if (a) add(rid(n, a) + 1, -im);
+    };
+    double dre = qr, dim = 0.0;
+#pragma unroll
+    for (int a = 0; a <= P; ++a) {
+        if (a > 0) {
+            const double c = SINGULAR ? 2.0 * a - 1.0 : 1.0 / (2.0 * a), x = c * ux, y = c * uy;
+            const double re = a > 1 ? x * dre - y * dim : x * dre;
+            dim = a > 1 ? x * dim + y * dre : y * dre;
+            dre = re;
+        }
+        put(a, a, dre, dim);
+        if (a + 1 <= P) {
+            const double z = SINGULAR ? (2.0 * a + 1.0) * uz : uz;
+            double p2re = dre, p2im = dim;
+            double p1re = z * dre, p1im = a ? z * dim : 0.0;
+            put(a + 1, a, p1re, p1im);
+#pragma unroll
+            for (int n = a + 2; n <= P; ++n) {
+                const double k = double(n * n - a * a);
+                const double zz = (SINGULAR ? 2.0 * n - 1.0 : (2.0 * n - 1.0) / k) * uz;
+                const double ww = (SINGULAR ? double((n - 1) * (n - 1) - a * a) : 1.0 / k) * w;
+                const double re = zz * p1re - ww * p2re;
+                p2re = p1re, p1re = re;
+                if (a) {
+                    const double im = zz * p1im - ww * p2im;
+                    p2im = p1im, p1im = im;
+                }
+                put(n, a, p1re, p1im);
+            }
+        }
+    }
+}
 
 // ---- per-point operators ----------------------------------------------------
 // P2M contribution of one body (mass q, scaled offset d from the box centre):

@@ -31,13 +31,33 @@ __device__ __forceinline__ int xcd_chunk_item() {
 }
 
 // ---- wave helpers -------------------------------------------------------------
+// Exchanges for the halving sum: afterwards a + b holds, in the lanes with bit M
+// clear, a's sum over the lane pair, and in the others b's. M = 32 and 16 swap
+// register halves (v_permlane32_swap, v_permlane16_swap).
+template <int M>
+__device__ __forceinline__ void swap_lanes(double& a, double& b) {
+    static_assert(M == 32 || M == 16, "lane swaps of gfx950");
+    const unsigned alo = __double2loint(a), ahi = __double2hiint(a), blo = __double2loint(b), bhi = __double2hiint(b);
+    if constexpr (M == 32) {
+        const auto lo = __builtin_amdgcn_permlane32_swap(alo, blo, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(ahi, bhi, false, false);
+        a = __hiloint2double(hi[0], lo[0]), b = __hiloint2double(hi[1], lo[1]);
+    } else {
+        const auto lo = __builtin_amdgcn_permlane16_swap(alo, blo, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(ahi, bhi, false, false);
+        a = __hiloint2double(hi[0], lo[0]), b = __hiloint2double(hi[1], lo[1]);
+    }
+}
+
 // Sums each of a lane's H register values over the wave by recursive halving:
 // at mask M = 32, 16, ..., 1 a lane keeps the lower ceil(H/2) of its values
 // when (lane & M) == 0, else the upper ones, and adds its partner's copy of
 // them. Every coefficient's total is one fixed sum tree (deterministic), and a
 // wave exchanges about H values instead of 6 H for H separate butterflies. On
 // return lane l holds the totals of coefficients first .. first + cnt - 1 in
-// v[0 .. cnt) (cnt <= 2 for H <= 128).
+// v[0 .. cnt) (cnt <= 2 for H <= 128). Three quarters of the exchanges are at
+// M = 32 and 16, where a register swap and the addition do one (three
+// instructions; two shuffles, four selects and the addition at the others).
 template <int H, int M>
 __device__ __forceinline__ void wave_halving_sum(double* v, int lane, int& first, int& cnt) {
     if constexpr (M >= 1) {
@@ -45,10 +65,15 @@ __device__ __forceinline__ void wave_halving_sum(double* v, int lane, int& first
         const bool up = (lane & M) != 0;
 #pragma unroll
         for (int q = 0; q < H2; ++q) {
-            const double lo = v[q];
-            const double hi = (H2 + q < H) ? v[H2 + q] : 0.0;
-            const double keep = up ? hi : lo;
-            v[q] = keep + __shfl_xor(up ? lo : hi, M, 64);
+            double lo = v[q];
+            double hi = (H2 + q < H) ? v[H2 + q] : 0.0;
+            if constexpr (M >= 16) {
+                swap_lanes<M>(lo, hi);
+                v[q] = lo + hi;
+            } else {
+                const double keep = up ? hi : lo;
+                v[q] = keep + __shfl_xor(up ? lo : hi, M, 64);
+            }
         }
         if (up) {
             first += H2;
@@ -65,8 +90,14 @@ __device__ __forceinline__ void wave_halving_sum(double* v, int lane, int& first
 // packed stream; each lane accumulates q conj(R(d)) (P2M, FmmExpansions3D.hpp:
 // 148-163) or q conj(S(d)) (P2L, AdaptiveFMM3D.hpp:117-128) of its bodies into
 // a register window of the S coefficients; the windows are then summed across
-// the wave by recursive halving (fixed order). Orders above 8 take two windows
-// (two passes over the stream) to bound registers.
+// the wave by recursive halving (fixed order). Orders above 8 take two or three
+// windows (passes over the stream) to bound registers.
+// Bound by FP64 VALU issue: a body costs 6 operations per complex harmonic and
+// one addition per coefficient (mass and 1/|d| enter the first harmonic, the
+// coefficients' scale follows the sum), a box the halving sum. All boxes,
+// P2L / P2M: 1M, p = 8 394 -> 334 / 145 -> 123 us, 300k, p = 12 324 -> 257 /
+// 113 -> 94, 700k, p = 4 120 -> 100 / 35 -> 33; at p = 16 the third window spills and they
+// stay where they were (287 -> 301 / 86 -> 88).
 //   KIND 0: targets = leaves, sources = the leaf's own bodies, Mhat = result.
 //   KIND 1: targets = boxes, sources = bodies of X(box) leaves, Lhat += result.
 //   KIND 2: as 1 into a separate array Lx (k_add_x then adds it to Lhat after
@@ -75,6 +106,20 @@ template <int S>
 constexpr int coef_windows() { return S <= 96 ? 1 : ((S + 127) / 128 > 2 ? (S + 127) / 128 : 2); }
 template <int S>
 constexpr int coef_window() { return (S + coef_windows<S>() - 1) / coef_windows<S>(); }
+
+template <int P>
+__constant__ FactScale<P> kFactScale = FactScale<P>();
+
+__device__ __forceinline__ double rounded_product(double a, double b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+// 1/sqrt(x) by two Newton steps from the 2^-24 hardware estimate.
+__device__ __forceinline__ double inv_sqrt(double x) {
+    double q = __builtin_amdgcn_rsq(x);
+    q = fma(q * 0.5, fma(-x * q, q, 1.0), q);
+    return fma(q * 0.5, fma(-x * q, q, 1.0), q);
+}
 
 // Where a coefficient goes in the packed multipoles of the FP64 M2L.
 template <int P>
@@ -176,8 +221,13 @@ __device__ __forceinline__ void accumulate_window(const TreeView& t, const int* 
                 auto add = [&](int k, double v) {
                     if (k >= C0 && k < C0 + CW) acc[k - C0] += v;
                 };
-                if (KIND == 0) p2m_point<P>(bm, dx, dy, dz, add);
-                else p2l_point<P>(bm, dx, dy, dz, add);
+                const double r2 = dx * dx + dy * dy + dz * dz;
+                if constexpr (KIND == 0) {
+                    point_terms<P, false>(bm, dx, dy, dz, r2, add);
+                } else {
+                    const double ir = inv_sqrt(r2), ir2 = ir * ir;
+                    point_terms<P, true>(bm * ir, dx * ir2, dy * ir2, dz * ir2, ir2, add);
+                }
             }
         }
     }
@@ -187,9 +237,12 @@ __device__ __forceinline__ void accumulate_window(const TreeView& t, const int* 
 #pragma unroll
     for (int k = 0; k < 2; ++k)
         if (k < cnt && C0 + first + k < S) {
-            if constexpr (KIND == 1) out[out_base + C0 + first + k] += acc[k];
-            else out[out_base + C0 + first + k] = acc[k];
-            if (KIND == 0 && packed) packed[kPack<P>.kpos[C0 + first + k]] = acc[k];
+            const int c = C0 + first + k;
+            // (rounded before it is added, so that KIND 1 and 2 give the same bits)
+            const double v = rounded_product(acc[k], KIND == 0 ? kFactScale<P>.inv[c] : kFactScale<P>.of[c]);
+            if constexpr (KIND == 1) out[out_base + c] += v;
+            else out[out_base + c] = v;
+            if (KIND == 0 && packed) packed[kPack<P>.kpos[c]] = v;
         }
 }
 
@@ -197,7 +250,7 @@ __device__ __forceinline__ void accumulate_window(const TreeView& t, const int* 
 // most X ranges hold too few bodies to occupy them).
 // Mp (KIND 0, may be null): the packed multipoles of the FP64 M2L, written too.
 template <int P, int KIND>
-__global__ void __launch_bounds__(64) k_accumulate(TreeView t, double* __restrict__ out, double* __restrict__ Mp) {
+__global__ void __launch_bounds__(64, 2) k_accumulate(TreeView t, double* __restrict__ out, double* __restrict__ Mp) {
     constexpr int S = nterms(P);
     constexpr int CW = coef_window<S>();
     __shared__ StreamLds sl;
@@ -255,8 +308,6 @@ constexpr int m2p_groups(int p) { return p <= 8 ? 32 : 16; }
 // Waves per SIMD that the registers are held to (p = 12: three 407, four 491 us).
 constexpr int m2p_waves(int p) { return p > 8 && p <= 12 ? 3 : 4; }
 __host__ __device__ inline int m2p_per_lane(int n) { return n > 14 ? 2 : 1; }
-template <int P>
-__constant__ FactScale<P> kFactScale = FactScale<P>();
 
 // Adds the field of one staged multipole m (box scale ih = 1/h) at R offsets d
 // (in units of h) from its centre: multipole_grad of afmm_math.h on the
@@ -269,10 +320,7 @@ __device__ __forceinline__ void m2p_pairs(const double* __restrict__ m, double i
     for (int r = 0; r < R; ++r) {
         const double x = d[r][0], y = d[r][1], z = d[r][2];
         const double r2 = x * x + y * y + z * z;
-        // 1/|v|: two Newton steps from the 2^-24 hardware estimate
-        double q = __builtin_amdgcn_rsq(r2);
-        q = fma(q * 0.5, fma(-r2 * q, q, 1.0), q);
-        q = fma(q * 0.5, fma(-r2 * q, q, 1.0), q);
+        const double q = inv_sqrt(r2);
         ir2[r] = q * q;
         ux[r] = x * ir2[r], uy[r] = y * ir2[r], uz[r] = z * ir2[r];
         dre[r] = q * (ih * ih);  // (the gradient's box scale; the potential takes it off again)
