@@ -307,8 +307,8 @@ typedef struct {
                                  at p = 7 and 8 tiles of up to 256 (16) or 128 (8) targets, no effect
                                  at other orders. Default 16 for FP64 at p <= 8 and p >= 14 and for
                                  bf16 at p <= 7, else 8 */
-    int32_t p2p_pair_bodies;  /* leaves with more bodies give each P2P lane two targets (default 32) */
-    int32_t p2p_min_group;    /* fewest lanes sharing one target's sources: 1, 2, 4, ..., 64 (default 8) */
+    int32_t p2p_pair_bodies;  /* leaves with more bodies give each P2P lane two targets (default 16) */
+    int32_t p2p_min_group;    /* fewest lanes sharing one target's sources: 1, 2, 4, ..., 64 (default 4) */
     int32_t p2p_schedule;     /* 1: persistent workgroups over the leaves sorted by work bin, largest
                                  first; 2: one workgroup per leaf in XCD-local chunks of tree order
                                  (the default) */

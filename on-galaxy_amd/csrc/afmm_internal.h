@@ -294,8 +294,11 @@ struct SideStream {
 // by work bin, largest first).
 struct Shapes {
     int m2l_waves = 16;  // 8 or 16
-    int p2p_pair_bodies = 32;
-    int p2p_min_group = 8;
+    // from a sweep over the benchmark's mergers, spheres and batch (P2P alone, us,
+    // 32 and 8 -> 16 and 4): 1M 670 -> 652, bf16 516 -> 507, 700k 499 -> 471,
+    // batch of 64 975 -> 939, 100k with potential 82 -> 76
+    int p2p_pair_bodies = 16;
+    int p2p_min_group = 4;
     int p2p_schedule = 0;
 };
 // The default M2L width of order p and precision mode prec (measured on the 1M

@@ -1295,8 +1295,8 @@ __global__ void __launch_bounds__(kT) k_add_x(int nb, int S, const int* __restri
 // sorted order) are streamed as one concatenated sequence in 64-body LDS
 // tiles: the ranges of up to kStreamChunk U boxes and their running body
 // offsets are staged in LDS once, and each lane finds the body of its tile
-// slot by binary search. Every lane holds R targets (R = 2 above 32 bodies,
-// else 1) of a lane group of T lanes (T = ceil(n_leaf / R), 8 <= T <= 64);
+// slot by binary search. Every lane holds R targets (R = 2 above 16 bodies,
+// else 1) of a lane group of T lanes (T = ceil(n_leaf / R), 4 <= T <= 64);
 // the wave's G = floor(64/T) groups take the tile's sources g, g+G, ... and
 // their partial sums are reduced in a fixed order (deterministic). The kernel
 // is (|d|^2 + eps^2)^{-3/2} from v_rsq_f64 refined by one Newton step; the
@@ -1357,7 +1357,7 @@ __device__ __forceinline__ void p2p_tile(const double* sx, const double* sy, con
             for (int r = 0; r < R; ++r) {
                 const double dx = xk - xi[r][0], dy = yk - xi[r][1], dz = zk - xi[r][2];
                 const bool self = MASK && j == ii[r];
-                const double r2 = self ? 1.0 : dx * dx + dy * dy + dz * dz + eps2;
+                const double r2 = self ? 1.0 : fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
                 const double m = self ? 0.0 : mk;
                 const double rin = rsqrt_f64(r2);
                 const double sc = m * (rin * rin * rin);
