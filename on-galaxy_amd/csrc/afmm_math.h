@@ -513,7 +513,7 @@ constexpr int src_row_of(int dx, int dy, int dz, int par) {
 }
 template <int NX>
 struct M2LSymSlots {
-    static constexpr int kMost = NX == 3 ? 56 : NX == 2 ? 100 : 178;
+    static constexpr int kMost = NX == 2 ? 100 : 178;
     int n = 0;
     short first[kMost] = {};
     short row[8][kMost][1 << NX] = {};

@@ -188,11 +188,7 @@ std::vector<double> sym_layout(const std::vector<double>& cm, int p) {
 }  // namespace
 
 std::vector<double> m2l_sym_layout(const std::vector<double>& cm, int p) {
-    switch (m2l_axes(p)) {
-        case 1: return sym_layout<1>(cm, p);
-        case 2: return sym_layout<2>(cm, p);
-        default: return sym_layout<3>(cm, p);
-    }
+    return m2l_axes(p) == 1 ? sym_layout<1>(cm, p) : sym_layout<2>(cm, p);
 }
 
 std::vector<double> m2l_a_layout(const std::vector<double>& cm, int S, int nmat) {

@@ -91,15 +91,15 @@ __constant__ M2LRoles<P, RS> kRoles = M2LRoles<P, RS>();
 
 // Waves of a workgroup; its tile holds at most 16 kM2LWaves CB / RS targets.
 constexpr int kM2LWaves = 8;
-// Pairs of k steps that a lane's source values are loaded ahead (a ring of
-// registers): what the registers of a wave leave (256, or 128 with two
-// workgroups per CU).
 // Units of 16 bytes of an operator chunk per thread, and those it holds at once.
 constexpr int m2l_stage_units(int p) {
     const int u = m2l_chunk_steps(p) * m2l_step(p) / 2, nt = kM2LWaves * 64;
     return (u + nt - 1) / nt;
 }
 constexpr int m2l_stage_regs(int p, int rs) { return rs > 1 ? m2l_stage_units(p) : (m2l_stage_units(p) + 1) / 2; }
+// Pairs of k steps that a lane's source values are loaded ahead (a ring of
+// registers): what the registers of a wave leave (256, or 128 with two
+// workgroups per CU).
 constexpr int m2l_depth(int p, int cb, int rs) {
     const M2LPlan t = make_m2l_plan(p);
     const int nm = 1 << m2l_axes(p);
