@@ -324,10 +324,9 @@ int afmm_get_shapes(const afmm_ctx* ctx, afmm_shapes* out);
  *   AFMM_OVERLAP_AUTO (the default): a second stream, shared by the process's
  *     contexts on that device, runs the upward pass beside the interaction-list
  *     build and P2P beside the far-field passes; with the bf16 or split-FP32
- *     M2L, and the FP64 one up to p = 8, from p = 14 and at p = 9-13 for up to
- *     500,000 bodies, the U/W/X lists, P2L, M2P and P2P
- *     run there beside M2L as well (their VALU work shares the SIMDs with its
- *     MFMAs);
+ *     M2L, and the FP64 one up to p = 8, from p = 12 and at p = 9-11 for up to
+ *     3,000,000 bodies, the U/W/X lists, P2L, M2P and P2P run there beside M2L
+ *     as well (their VALU work shares the SIMDs with its MFMAs);
  *   AFMM_OVERLAP_BESIDE_M2L: the latter schedule in every form, with P2P
  *     beside M2L too (the automatic schedule starts P2P after the bf16 M2L);
  *   AFMM_OVERLAP_IN_ORDER: the former (lists, P2L and M2P in order before M2L).

@@ -318,12 +318,10 @@ class AdaptiveFMM3D:
         """Two-stream overlap (afmm_set_overlap): True or OVERLAP_AUTO (the
         default: the upward pass beside the list build, P2P beside the
         far-field passes, and with the bf16 or split-FP32 M2L, or FP64 up to
-        p = 8, from p = 14 and at p = 9-13 for up to 500,000 bodies, the
-        lists, P2L, M2P and P2P beside M2L),
-        OVERLAP_BESIDE_M2L,
-        OVERLAP_IN_ORDER, or
-        False / OVERLAP_OFF (one stream, in order). Results are the same bits
-        in every mode."""
+        p = 8, from p = 12 and at p = 9-11 for up to 3,000,000 bodies, the
+        lists, P2L, M2P and P2P beside M2L), OVERLAP_BESIDE_M2L,
+        OVERLAP_IN_ORDER, or False / OVERLAP_OFF (one stream, in order).
+        Results are the same bits in every mode."""
         mode = OVERLAP_AUTO if enable is True else OVERLAP_OFF if enable is False else int(enable)
         self._check(self.lib.afmm_set_overlap(self.ctx, mode))
 

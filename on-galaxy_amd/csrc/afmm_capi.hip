@@ -64,9 +64,9 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
 // The evaluation of nsys systems (concatenated device arrays: pos AoS n x 3,
 // mass n; system q = bodies [sys_off[q], sys_off[q+1])) into acc (AoS, input
 // order) and optionally phi. G and eps per system (host arrays).
-// FP64 at p = 9-13: the most bodies for which the automatic schedule runs the
+// FP64 at p = 9-11: the most bodies for which the automatic schedule runs the
 // list, P2L, M2P and P2P passes beside M2L.
-constexpr int64_t kBesideMaxBodiesMidOrders = 500000;
+constexpr int64_t kBesideMaxBodiesMidOrders = 3000000;
 
 int afmm::eval_forest(afmm_ctx* c, int nsys, const int* sys_off, const double* G, const double* eps, const double* pos,
                 const double* mass, double* acc, double* phi) {
@@ -99,17 +99,18 @@ int afmm::eval_forest(afmm_ctx* c, int nsys, const int* sys_off, const double* G
     // P2L, M2P and P2P run on the second stream beside it, after the upward
     // pass: their VALU work shares the SIMDs with the MFMA-bound M2L, and the
     // lists' size readback synchronises the second stream only. The
-    // automatic choice, from the merger at 16k-1M bodies: beside for the bf16
-    // (1M, p = 8: 4.34 -> 4.13 ms) and split-FP32 (7.75 -> 7.54 ms) forms, and
-    // for FP64 up to p = 8 (1M: 5.79 -> 5.67 ms at p = 8, 2.51 -> 2.45 ms at
-    // p = 4; 16k: 1.48 -> 1.26 ms at p = 8) and from p = 14 (16-wave
-    // row-split M2L: 44.8 -> 41.9 ms at p = 14, 78.8 -> 73.8 ms at p = 16);
-    // FP64 at p = 9-13 beside up to 500k bodies (p = 12: 7.26 -> 7.00 ms at
-    // 16k, 13.7 -> 13.0 ms at 400k) and in order above, where the longer M2L
-    // loses more beside the VALU passes than they save (1M, p = 12: 23.9 ms
-    // against 27.5 ms beside).
+    // automatic choice, from mergers and spheres at 16k-5M bodies (ms per
+    // evaluation, in order -> beside): beside for the bf16 (1M, p = 8: 4.02 ->
+    // 3.88) and split-FP32 forms and for FP64 up to p = 8 (16k p = 8: 1.29 ->
+    // 1.13; 1M: 2.91 -> 2.85 at p = 6, 4.17 -> 4.18 at p = 8; 4M p = 8: 15.1 ->
+    // 14.4) and from p = 12 (1M p = 12: 10.17 -> 9.84, 600k p = 14: 14.4 ->
+    // 11.0, 4M p = 12: 38.3 -> 36.7); FP64 at p = 9-11 beside up to 3M bodies
+    // (1M p = 9: 5.86 -> 5.47, 2M p = 9: 10.8 -> 10.1, 3M p = 10: 19.0 -> 18.9)
+    // and in order above (4M: 20.67 against 20.91 beside at p = 9, 25.0
+    // against 25.2 at p = 10, p = 11: 27.6 against 28.0), where every pass
+    // fills the GPU and M2L loses more than the VALU passes save.
     const bool bf16_m2l = m2l_form(c->prm.precision) == kPrecMixedBf16;
-    const bool auto_beside = m2l_form(c->prm.precision) != kPrecFP64 || c->prm.p <= 8 || c->prm.p >= 14 ||
+    const bool auto_beside = m2l_form(c->prm.precision) != kPrecFP64 || c->prm.p <= 8 || c->prm.p >= 12 ||
                              n <= kBesideMaxBodiesMidOrders;
     const bool lists_beside = split && !c->use_graph &&
                               (c->overlap_mode == AFMM_OVERLAP_BESIDE_M2L ||
