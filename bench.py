@@ -523,9 +523,9 @@ def main():
     S = (args.p + 1) ** 2
     m2l_flops = 2.0 * S * S * st["n_v"]
     achieved = m2l_flops / (avg["m2l"] * 1e-3) / 1e12
-    roofline = {"kernel": "M2L (k_m2l_mfma, FP64 MFMA)", "bound": "mfma", "achieved": achieved,
+    roofline = {"kernel": "M2L (k_m2l_fp64, FP64 MFMA)", "bound": "mfma", "achieved": achieved,
                 "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s", "frac": achieved / PEAK_FP64_TFLOPS,
-                "traffic": measured_traffic("k_m2l_mfma_fp64"),
+                "traffic": measured_traffic("k_m2l_fp64"),
                 "traffic_source": "profiles/m2l_traffic_merger1M_p8.md (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE)",
                 "algorithmic_per_launch": f"2*S^2*|V| = 2*{S}^2*{st['n_v']} = {m2l_flops:.4e} flop"}
 
@@ -538,7 +538,7 @@ def main():
     # starts beside M2L and the two share the CUs for part of M2L's duration
     alone = m2l_flops / (seq_avg["m2l"] * 1e-3) / 1e12
     roofline["alone"] = {"ms": seq_avg["m2l"], "achieved": alone, "frac": alone / PEAK_FP64_TFLOPS,
-                         "note": "k_m2l_mfma in the one-stream run (afmm_set_overlap 0), no other kernel beside it"}
+                         "note": "k_m2l_fp64 in the one-stream run (afmm_set_overlap 0), no other kernel beside it"}
 
     # PCIe-inclusive drop-in semantics (host arrays in and out), reported aside:
     # median of 5 after a warm-up

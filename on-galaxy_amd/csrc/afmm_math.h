@@ -440,6 +440,9 @@ AFMM_HD constexpr int m2l_kb(int S) { return (S + 3) / 4; }
 // 16 bytes hold one k of both steps of a pair. Rows: 16-row blocks per class
 // (v_mfma_f64_16x16x4) and its remainder of at most 12 rows in quads of 4
 // (v_mfma_f64_4x4x4, a quarter of the time).
+// NX = 2 from p = 4: below, a class has too few rows and columns to fill its
+// quads and steps of 4, which takes what the fewer products save (1M merger,
+// M2L us, NX = 1 and 2: p = 2 174 and 188, p = 3 249 and 254).
 constexpr int m2l_axes(int p) { return p >= 4 ? 2 : 1; }
 constexpr int kPlanSteps = kMaxTerms / 4 + 8, kPlanBlocks = 24, kPlanQuads = 24;
 struct M2LPlan {
@@ -494,7 +497,7 @@ constexpr int m2l_step(int p) { return make_m2l_plan(p).nb * 64 + make_m2l_plan(
 
 // Workgroups that share a CU: two where two double-buffered operators fit its
 // LDS. Else one, whose waves own two 16-target columns where their accumulators
-// fit the registers.
+// fit the registers. 700k merger, p = 4: one workgroup 461 us, two 400.
 constexpr int m2l_workgroups(int p) { return p <= 6 ? 2 : 1; }
 constexpr int m2l_columns(int p) { return p == 7 || p == 8 ? 2 : 1; }
 
