@@ -147,12 +147,13 @@ void worker_loop(afmm_server* sv, Worker* w);
 
 // Footprint estimate at leaf capacity cap: resident arrays 80 B/body; batch
 // copies, keys, sort and sorted bodies ~420 B/body; per box the two
-// expansions (2 S doubles) and the lists (~1.3 KB). Boxes number about
+// expansions and the multipoles in M2L's order (3 S doubles) and the lists
+// (~1.3 KB). Boxes number about
 // 4 n / cap + 64 (n / 16 at capacity 64; measured n / 22 on the merger).
 int64_t job_bytes_cap(int64_t n, int32_t p, int32_t cap) {
     const int64_t S = (int64_t)(p + 1) * (p + 1);
     const int64_t boxes = 4 * n / std::max<int32_t>(cap, 1) + 64;
-    return n * 500 + boxes * (16 * S + 1300);
+    return n * 500 + boxes * (24 * S + 1300);
 }
 
 // The worker of order p, created with its context on first use (caller holds
